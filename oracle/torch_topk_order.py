@@ -22,16 +22,19 @@ algorithms (libstdc++'s published implementation: median-of-three pivot moved
 to the front, unguarded Hoare partition, insertion sort below 17 (sort) or 4
 (select) elements, heap fallbacks at a depth limit of 2*floor(log2 n)).
 
-Two restatements live here:
+Three restatements live here:
 
 * ``topk_order_seq`` follows those algorithms step by step;
-* ``topk_order_wave`` is the form the HIP kernel runs on one wavefront
-  (vsa-lm_amd/csrc/bolt3_chain.hip, ``tie_order_wave``): each Hoare partition
-  is computed in one pass from the ranks of its left and right stops, the sort's
-  ranges are partitioned independently, and the final insertion sort is a
-  stable rank.
+* ``topk_order_wave`` computes each Hoare partition in one pass from the ranks
+  of its left and right stops, partitions the sort's ranges independently, and
+  makes the final insertion sort a stable rank;
+* ``topk_order_levels`` is the form the HIP kernel runs on one wavefront
+  (vsa-lm_amd/csrc/bolt3_chain.hip, ``tie_order_wave``): the same partitions on
+  dense keys (the number of elements strictly before an element), every range of
+  a level of the sort's recursion at once, and the insertion sort as the dense key
+  plus the number of equal elements at lower positions.
 
-tests/test_tie_order.py pins both against torch.topk itself on tie-heavy
+tests/test_tie_order.py pins them against torch.topk itself on tie-heavy
 arrays (NaN, -0/+0, long runs of equal values, both directions, both library
 paths).
 """
@@ -265,6 +268,44 @@ def topk_order_wave(values, k: int, largest: bool = True) -> tuple[list[int], bo
             stack += [(cut, sl, d - 1), (sf, cut, d - 1)]
     _stable(key, idx, 0, ks)
     return [int(i) for i in idx[:k]], limit
+
+
+def topk_order_levels(values, k: int, largest: bool = True) -> tuple[list[int], bool]:
+    """The kernel's restatement, level by level.  Returns (indices, depth_limit_reached)."""
+    n = len(values)
+    if k <= 0:
+        return [], False
+    if 64 * k <= n:
+        return topk_order_seq(values, k, largest), False
+    full = [order_key(v, largest) for v in values]
+    key = np.array([sum(o < c for o in full) for c in full], dtype=np.int64)     # dense keys
+    idx = np.arange(n)
+    f, l, depth = 0, n, 2 * _lg(n)
+    while l - f > SELECT_THRESHOLD:
+        if depth == 0:
+            return [int(i) for i in idx[:k]], True
+        depth -= 1
+        cut = _partition_wave(key, idx, f, l)
+        f, l = (cut, l) if cut <= k - 1 else (f, cut)
+    _stable(key, idx, f, l)
+    ks = k - 1
+    ranges, depth = [(0, ks)], 2 * _lg(ks) if ks > 1 else 0
+    while any(b - a > SORT_THRESHOLD for a, b in ranges):
+        if depth == 0:
+            return [int(i) for i in idx[:k]], True
+        depth -= 1
+        level = []
+        for a, b in ranges:            # disjoint: the kernel partitions them in one pass
+            if b - a > SORT_THRESHOLD:
+                cut = _partition_wave(key, idx, a, b)
+                level += [(a, cut), (cut, b)]
+            else:
+                level.append((a, b))
+        ranges = level
+    out = [int(idx[k - 1])] * k
+    for p in range(ks):
+        out[int(key[p]) + int((key[:p] == key[p]).sum())] = int(idx[p])
+    return out, False
 
 
 def tie_in_prefix(sorted_values, n: int) -> bool:

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 import torch
 
-from oracle.torch_topk_order import tie_in_prefix, topk_order_seq, topk_order_wave
+from oracle.torch_topk_order import tie_in_prefix, topk_order_levels, topk_order_seq, topk_order_wave
 
 
 def _case(t: int, rng: random.Random):
@@ -60,6 +60,19 @@ def test_restatement_matches_torch_topk(form):
     assert not bad, bad[:5]
 
 
+def test_level_form_matches_torch_topk():
+    """The form the kernel runs: every range of a level of the sort's recursion at once."""
+    rng = random.Random(11)
+    bad = []
+    for t in range(1500):
+        v, k, largest = _case(t, rng)
+        got, limit = topk_order_levels(v.tolist(), k, largest)
+        assert not limit, (t, len(v), k)
+        if got != torch.topk(torch.from_numpy(v), k, largest=largest)[1].tolist():
+            bad.append((t, len(v), k, largest))
+    assert not bad, bad[:5]
+
+
 def test_slot_decision_shapes():
     """The kernel's calls: candidates (n = l tokens, k = min(l, 128), largest) and keep values
     (n = 128 slots, k = min(l, 128), smallest), with runs of equal keeps (mutual nearest slots
@@ -77,6 +90,8 @@ def test_slot_decision_shapes():
         for vals, largest in ((cand, True), (keep, False)):
             want = torch.topk(torch.from_numpy(vals), kc, largest=largest)[1].tolist()
             assert topk_order_wave(vals.tolist(), kc, largest)[0] == want
+            if t < 60:
+                assert topk_order_levels(vals.tolist(), kc, largest)[0] == want
 
 
 def test_tie_in_prefix():

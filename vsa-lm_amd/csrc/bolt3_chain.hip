@@ -41,7 +41,6 @@ namespace b3 {
 
 constexpr int S = 128;     // attractor slots
 constexpr int LMAX = 256;  // tokens per consolidation step
-constexpr int TIE_STACK = 32;  // pending ranges of the tie-order sort
 constexpr int DT = 512;    // decide_kernel threads
 constexpr int DWAVES = DT / WAVE;
 constexpr int MT = 256;    // gersh_kernel / mres_kernel threads
@@ -117,10 +116,8 @@ struct DecSmem {
     } mg;
     struct { float mx[2][S]; int nan[2][S]; } kp;
     struct { alignas(16) uint64_t a[LMAX]; alignas(16) uint64_t b[S]; } ok;
-    struct {   // tie order (one wavefront per ordering): packed elements, stop positions, ranges
-      alignas(16) uint64_t e[2][LMAX];
-      int pr[2][LMAX + 1];
-      int stk[2][3 * TIE_STACK];
+    struct {   // tie order (one wavefront per ordering): packed elements, swapped pairs by rank
+      uint32_t e[2][LMAX + 1], xl[2][LMAX + 1], xr[2][LMAX + 1];
     } to;
   } u;
 };
@@ -309,132 +306,116 @@ __device__ __forceinline__ int count_below(const uint64_t* keys, int i0, int i1,
 //    partitions, and insertion sort is stable, so a stable rank of the whole sorted range
 //    gives the final order;
 //  * partial_sort (k <= 4) runs its heap steps uniformly on the whole wavefront.
-// Elements are packed as (key << 32 | source index) with a 32-bit key that is lowest for the
-// element that comes first (NaN first when largest, last otherwise; -0 equals +0, as in a float
-// comparison).  A depth limit reached (heap fallback of the library, not restated) sets bit 0
-// of the returned flags.
+// Elements are packed as (lt << 8 | source index), lt = the number of elements strictly before
+// them (n <= 256), which orders as the values do (NaN first when largest, last otherwise; -0
+// equals +0, as in a float comparison).  Position p of the array lives in register p / 64 of lane
+// p % 64.  A partition takes two LDS round trips (the four elements the pivot is chosen from, the
+// exchange of the swapped pairs), and the ranges of the sort, which do not touch each other, are
+// partitioned all at once, a level of the recursion at a time: each lane counts the stops of its
+// own range from ballots masked to it.  The first steady step of a sequence, whose slots all hold
+// the same utility, orders its 128 slots this way; the chain of levels bounds it: 14 us (HD = 128)
+// where one range after the other, with its elements in LDS as 64-bit keys, took 41 us.
+// A depth limit reached (heap fallback of the library, not restated) sets bit 0 of the returned
+// flags.
 __device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-__device__ __forceinline__ uint32_t tie_key(float v, bool largest) {
-  const uint32_t k = ord_key(v + 0.0f);
-  return largest ? ~k : k;
-}
-__device__ __forceinline__ uint32_t pk_key(uint64_t e) { return (uint32_t)(e >> 32); }
+__device__ __forceinline__ uint32_t pk_key(uint32_t e) { return e >> 8; }
 
-// Median-of-three move and Hoare partition of e[f, l) (l - f > 3); returns the cut.
-__device__ int tie_partition(uint64_t* e, int* pr, int f, int l, int lane, int& flags) {
-  const int a = f + 1, b = f + (l - f) / 2, c = l - 1;
-  const uint32_t ka = pk_key(e[a]), kb = pk_key(e[b]), kc = pk_key(e[c]);
-  int t;
-  if (ka < kb) t = kb < kc ? b : (ka < kc ? c : a);
-  else t = ka < kc ? a : (kb < kc ? c : b);
-  const uint64_t ef = e[f], et = e[t];
-  wave_lds_fence();
-  if (lane == 0) {
-    e[f] = et;
-    e[t] = ef;
-  }
-  wave_lds_fence();
-  const uint32_t piv = pk_key(et);
-  const unsigned long long below = (1ull << lane) - 1ull;
-  uint64_t x[4];
-  bool lf[4], rf[4];
-  unsigned long long bl[4], br[4];
-  int tot_r = 0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int q = a + lane + WAVE * j;
-    x[j] = 0ull;
-    if (q < l) x[j] = e[q];
-    const uint32_t k = pk_key(x[j]);
-    lf[j] = q < l && k >= piv;
-    rf[j] = q < l && k <= piv;
-    bl[j] = __ballot(lf[j]);
-    br[j] = __ballot(rf[j]);
-    tot_r += __popcll(br[j]);
-  }
-  int cl = 0, cr = 0, m = 0;
-  int rank_l[4], above[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    rank_l[j] = cl + __popcll(bl[j] & below) + 1;
-    above[j] = tot_r - (cr + __popcll(br[j] & below) + (rf[j] ? 1 : 0));   // R stops above q
-    cl += __popcll(bl[j]);
-    cr += __popcll(br[j]);
-    m += __popcll(__ballot(lf[j] && above[j] >= rank_l[j]));
-  }
-  const int tot_l = cl;
-  // pr[i] = position of the i-th right stop (i <= m); pr[0] = the (m+1)-th left stop
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int q = a + lane + WAVE * j;
-    if (rf[j] && above[j] + 1 <= m) pr[above[j] + 1] = q;
-    if (lf[j] && rank_l[j] == m + 1) pr[0] = q;
-  }
-  wave_lds_fence();
-  uint64_t y[4];
-  int pp[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    pp[j] = 0;
-    y[j] = 0ull;
-    if (lf[j] && rank_l[j] <= m) {
-      pp[j] = pr[rank_l[j]];
-      y[j] = e[pp[j]];
-    }
-  }
-  const int l_next = tot_l > m ? pr[0] : INT_MAX;
-  const int r_m = m > 0 ? pr[m] : INT_MAX;
-  wave_lds_fence();
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (lf[j] && rank_l[j] <= m) {
-      e[a + lane + WAVE * j] = y[j];
-      e[pp[j]] = x[j];
-    }
-  }
-  wave_lds_fence();
-  int cut = min(l_next, r_m);
-  if (cut == INT_MAX) {   // no left stop at all: cannot happen after a median-of-three move
-    flags |= 1;
-    cut = l;
-  }
-  return __builtin_amdgcn_readfirstlane(cut);
+// Bits of chunk j (positions 64 j ..) that lie in the range [f, l).
+__device__ __forceinline__ unsigned long long range_bits(int f, int l, int j) {
+  const int lo = min(max(f - WAVE * j, 0), WAVE), hi = min(max(l - WAVE * j, 0), WAVE);
+  const unsigned long long below_hi = hi == WAVE ? ~0ull : (1ull << hi) - 1ull;
+  const unsigned long long below_lo = lo == WAVE ? ~0ull : (1ull << lo) - 1ull;
+  return below_hi & ~below_lo;
 }
 
-// Stable order of e[f, l) by key, in place (insertion sort's result).
-__device__ void tie_stable_range(uint64_t* e, int f, int l, int lane) {
-  uint64_t x[4];
-  int r[4];
+// One median-of-three move and Hoare partition of every active range at once.  x: the elements
+// (position lane + 64 j), e: the same in LDS, [f, l): the range of each position, on: whether
+// that range (l - f > 3) is partitioned.  Returns each range's cut in cut[].
+template <int NJ>
+__device__ void tie_level(uint32_t (&x)[NJ], const int (&f)[NJ], const int (&l)[NJ], const bool (&on)[NJ],
+                          int (&cut)[NJ], uint32_t* e, uint32_t* xl, uint32_t* xr, int lane, int& flags) {
+  bool lf[NJ], rf[NJ];
+  unsigned long long bl[NJ], br[NJ];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int i = f + lane + WAVE * j;
-    x[j] = 0ull;
-    r[j] = 0;
-    if (i < l) x[j] = e[i];
-  }
-  for (int t = f; t < l; ++t) {
-    const uint64_t y = e[t];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = f + lane + WAVE * j;
-      r[j] += (pk_key(y) < pk_key(x[j]) || (pk_key(y) == pk_key(x[j]) && t < i)) ? 1 : 0;
+  for (int i = 0; i < NJ; ++i) {
+    const int p = lane + WAVE * i;
+    lf[i] = rf[i] = false;
+    if (on[i]) {
+      const int pa = f[i] + 1, pb = f[i] + (l[i] - f[i]) / 2, pc = l[i] - 1;
+      const uint32_t ea = e[pa], eb = e[pb], ec = e[pc], ef = e[f[i]];
+      const uint32_t ka = pk_key(ea), kb = pk_key(eb), kc = pk_key(ec);
+      int t;
+      if (ka < kb) t = kb < kc ? pb : (ka < kc ? pc : pa);
+      else t = ka < kc ? pa : (kb < kc ? pc : pb);
+      const uint32_t et = t == pa ? ea : (t == pb ? eb : ec);
+      x[i] = p == f[i] ? et : (p == t ? ef : x[i]);
+      lf[i] = p > f[i] && pk_key(x[i]) >= pk_key(et);
+      rf[i] = p > f[i] && pk_key(x[i]) <= pk_key(et);
     }
+    bl[i] = __ballot(lf[i]);
+    br[i] = __ballot(rf[i]);
+  }
+  // rank_l: the position's number among its range's left stops (from 1); above: the right stops
+  // above it; the pair (i-th left, i-th right stop) swaps while the left one lies below
+  int rank_l[NJ], above[NJ], m[NJ];
+  unsigned long long bm[NJ];
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    const int p = lane + WAVE * i;
+    rank_l[i] = above[i] = 0;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      rank_l[i] += __popcll(bl[j] & range_bits(f[i], p + 1, j));
+      above[i] += __popcll(br[j] & range_bits(p + 1, l[i], j));
+    }
+    bm[i] = __ballot(lf[i] && above[i] >= rank_l[i]);
+  }
+  bool sl[NJ], sr[NJ];
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    m[i] = 0;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) m[i] += __popcll(bm[j] & range_bits(f[i], l[i], j));
+    sl[i] = lf[i] && rank_l[i] <= m[i];
+    sr[i] = rf[i] && above[i] + 1 <= m[i];
+    if (sl[i]) xl[f[i] + rank_l[i]] = x[i];
+    if (sr[i]) xr[f[i] + above[i] + 1] = x[i];
   }
   wave_lds_fence();
+  unsigned long long bn[NJ], bq[NJ];   // each range's first unswapped left stop, last swapped right stop
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if (f + lane + WAVE * j < l) e[f + r[j]] = x[j];
+  for (int i = 0; i < NJ; ++i) {
+    if (sl[i]) x[i] = xr[f[i] + rank_l[i]];
+    else if (sr[i]) x[i] = xl[f[i] + above[i] + 1];
+    bn[i] = __ballot(lf[i] && rank_l[i] == m[i] + 1);
+    bq[i] = __ballot(rf[i] && above[i] + 1 == m[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    int c = INT_MAX;
+#pragma unroll
+    for (int j = NJ - 1; j >= 0; --j) {
+      const unsigned long long b = (bn[j] | bq[j]) & range_bits(f[i], l[i], j);
+      if (b) c = WAVE * j + __builtin_ctzll(b);
+    }
+    if (on[i] && c == INT_MAX) {   // no left stop at all: cannot happen after a median-of-three move
+      flags |= 1;
+      c = l[i];
+    }
+    cut[i] = c;
+    if (on[i]) e[lane + WAVE * i] = x[i];
+  }
   wave_lds_fence();
 }
 
 // Heap steps of the library's partial_sort, executed alike by every lane (k <= 4, so the heap
 // is a few LDS words; the same value is stored by every lane).
-__device__ __forceinline__ void heap_put(uint64_t* e, int i, uint64_t v) {
+__device__ __forceinline__ void heap_put(uint32_t* e, int i, uint32_t v) {
   e[i] = v;
   wave_lds_fence();
 }
-__device__ void heap_adjust(uint64_t* e, int hole, int len, uint64_t v) {
+__device__ void heap_adjust(uint32_t* e, int hole, int len, uint32_t v) {
   const int top = hole;
   int child = hole;
   while (child < (len - 1) / 2) {
@@ -456,17 +437,42 @@ __device__ void heap_adjust(uint64_t* e, int hole, int len, uint64_t v) {
   }
   heap_put(e, hole, v);
 }
-__device__ void heap_pop(uint64_t* e, int len, int res) {
-  const uint64_t v = e[res];
+__device__ void heap_pop(uint32_t* e, int len, int res) {
+  const uint32_t v = e[res];
   heap_put(e, res, e[0]);
   heap_adjust(e, 0, len, v);
 }
 
-// torch.topk's order of the k first elements of e[0, n) (packed with tie_key): source indices
-// into out[0, k).  One wavefront; pr holds LMAX + 1 ints, stk 3 * TIE_STACK ints.
-__device__ int tie_order_wave(uint64_t* e, int* pr, int* stk, int n, int k, int* out, int lane) {
+// torch.topk's order of the first k of n values (k <= n <= 64 NJ), given sorted[0, n) (the values
+// in rank order) and src[0, n) (their source indices): source indices into src[0, k).  One
+// wavefront; e, xl and xr hold LMAX + 1 words each.
+template <int NJ>
+__device__ int tie_order_wave(const float* sorted, int* src, uint32_t* e, uint32_t* xl, uint32_t* xr, int n, int k,
+                              int lane) {
   int flags = 0;
   if (k <= 0) return 0;
+  {   // lt: the first rank of the run of equal values that a rank lies in
+    unsigned long long first[NJ];
+    int sj[NJ];
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int r = lane + WAVE * i;
+      const bool in = r < n;
+      sj[i] = in ? src[r] : 0;
+      first[i] = __ballot(in && (r == 0 || ord_key(sorted[r] + 0.0f) != ord_key(sorted[r - 1] + 0.0f)));
+    }
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int r = lane + WAVE * i;
+      int lt = 0;
+#pragma unroll
+      for (int j = 0; j <= i; ++j) {
+        const unsigned long long b = first[j] & range_bits(0, r + 1, j);
+        if (b) lt = WAVE * j + 63 - __builtin_clzll(b);
+      }
+      if (r < n) e[sj[i]] = ((uint32_t)lt << 8) | (uint32_t)sj[i];
+    }
+  }
   wave_lds_fence();
   if (k * 64 <= n) {
     if (k >= 2)
@@ -480,58 +486,133 @@ __device__ int tie_order_wave(uint64_t* e, int* pr, int* stk, int n, int k, int*
       --last;
       heap_pop(e, last, last);
     }
-  } else {
-    // nth_element at k - 1
-    int f = 0, l = n, depth = 2 * (31 - __clz(n));
-    while (l - f > 3) {
-      if (depth == 0) {
-        flags |= 1;
-        break;
-      }
-      --depth;
-      const int cut = tie_partition(e, pr, f, l, lane, flags);
-      if (cut <= k - 1) f = cut;
-      else l = cut;
-    }
-    tie_stable_range(e, f, l, lane);
-    // sort of [0, k - 1): the ranges above 16 elements are partitioned, the rest is left in
-    // place for the final insertion sort
-    const int ks = k - 1;
-    if (ks > 16) {
-      if (lane == 0) {
-        stk[0] = 0;
-        stk[1] = ks;
-        stk[2] = 2 * (31 - __clz(ks));
-      }
-      wave_lds_fence();
-      int sp = 1;
-      while (sp > 0) {
-        --sp;
-        const int sf = stk[3 * sp], sl = stk[3 * sp + 1], d = stk[3 * sp + 2];
-        wave_lds_fence();
-        if (sl - sf <= 16) continue;
-        if (d == 0 || sp + 2 > TIE_STACK) {
-          flags |= 1;
-          continue;
-        }
-        const int cut = tie_partition(e, pr, sf, sl, lane, flags);
-        if (lane == 0) {
-          stk[3 * sp + 0] = cut;
-          stk[3 * sp + 1] = sl;
-          stk[3 * sp + 2] = d - 1;
-          stk[3 * sp + 3] = sf;
-          stk[3 * sp + 4] = cut;
-          stk[3 * sp + 5] = d - 1;
-        }
-        sp += 2;
-        wave_lds_fence();
-      }
-    }
-    tie_stable_range(e, 0, ks, lane);
+    for (int i = lane; i < k; i += WAVE) src[i] = (int)(e[i] & 255u);
+    wave_lds_fence();
+    return flags;
   }
-  for (int i = lane; i < k; i += WAVE) out[i] = (int)(uint32_t)e[i];
+  uint32_t x[NJ];
+  int sf[NJ], sl[NJ], cut[NJ];
+  bool on[NJ];
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) x[i] = lane + WAVE * i < n ? e[lane + WAVE * i] : 0u;
+  // nth_element at k - 1
+  int f = 0, l = n, depth = 2 * (31 - __clz(n));
+  while (l - f > 3) {
+    if (depth == 0) {
+      flags |= 1;
+      break;
+    }
+    --depth;
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int p = lane + WAVE * i;
+      sf[i] = f;
+      sl[i] = l;
+      on[i] = p >= f && p < l;
+    }
+    tie_level<NJ>(x, sf, sl, on, cut, e, xl, xr, lane, flags);
+    // every lane's range is [f, l) here, so any lane's cut is the range's
+    int c = l;
+#pragma unroll
+    for (int i = NJ - 1; i >= 0; --i) {
+      const unsigned long long b = __ballot(on[i]);
+      if (b) c = __builtin_amdgcn_readlane(cut[i], __builtin_ctzll(b));
+    }
+    if (c <= k - 1) f = c;
+    else l = c;
+  }
+  if (l - f <= 3) {   // the last elements by insertion sort (stable)
+    int to[NJ];
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int p = lane + WAVE * i;
+      to[i] = f;
+      for (int q = f; q < l; ++q) to[i] += pk_key(e[q]) < pk_key(x[i]) || (pk_key(e[q]) == pk_key(x[i]) && q < p);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int p = lane + WAVE * i;
+      if (p >= f && p < l) e[to[i]] = x[i];
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int p = lane + WAVE * i;
+      if (p >= f && p < l) x[i] = e[p];
+    }
+  }
+  // sort of [0, k - 1): the ranges above 16 elements are partitioned, the rest is left to the
+  // final insertion sort
+  const int ks = k - 1;
+  depth = ks > 1 ? 2 * (31 - __clz(ks)) : 0;
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    sf[i] = 0;
+    sl[i] = ks;
+  }
+  for (;; --depth) {
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int p = lane + WAVE * i;
+      on[i] = p >= sf[i] && p < sl[i] && sl[i] - sf[i] > 16;
+      any |= __ballot(on[i]) != 0;
+    }
+    if (!any) break;
+    if (depth == 0) {
+      flags |= 1;
+      break;
+    }
+    tie_level<NJ>(x, sf, sl, on, cut, e, xl, xr, lane, flags);
+#pragma unroll
+    for (int i = 0; i < NJ; ++i)
+      if (on[i]) {
+        if (lane + WAVE * i >= cut[i]) sf[i] = cut[i];
+        else sl[i] = cut[i];
+      }
+  }
+  // insertion sort is stable: an element ends after those strictly before it (all of them lie in
+  // [0, k - 1)) and the equal ones at lower positions
+  {
+    unsigned long long eq[NJ][NJ];   // [i][j]: positions of chunk j equal to the lane's element of chunk i
+#pragma unroll
+    for (int i = 0; i < NJ; ++i)
+#pragma unroll
+      for (int j = 0; j <= i; ++j) eq[i][j] = range_bits(0, min(ks, lane + WAVE * i), j);
+#pragma unroll
+    for (int b = 8; b < 16; ++b) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const unsigned long long ones = __ballot((x[j] >> b) & 1u);
+#pragma unroll
+        for (int i = j; i < NJ; ++i) eq[i][j] &= ((x[i] >> b) & 1u) ? ones : ~ones;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) {
+      const int p = lane + WAVE * i;
+      int to = (int)pk_key(x[i]);
+#pragma unroll
+      for (int j = 0; j <= i; ++j) to += __popcll(eq[i][j]);
+      if (p < ks) src[to] = (int)(x[i] & 255u);
+      if (p == ks) src[p] = (int)(x[i] & 255u);
+    }
+  }
   wave_lds_fence();
   return flags;
+}
+
+// The same for up to LMAX values: two positions per lane where they suffice.  The other form stays
+// out of line: its registers beside the next step's prefetched tile would not fit.
+__device__ __noinline__ int tie_order_long(const float* sorted, int* src, uint32_t* e, uint32_t* xl, uint32_t* xr,
+                                           int n, int k, int lane) {
+  return tie_order_wave<LMAX / WAVE>(sorted, src, e, xl, xr, n, k, lane);
+}
+__device__ __forceinline__ int tie_order(const float* sorted, int* src, uint32_t* e, uint32_t* xl, uint32_t* xr, int n,
+                                         int k, int lane) {
+  return n <= 2 * WAVE ? tie_order_wave<2>(sorted, src, e, xl, xr, n, k, lane)
+                       : tie_order_long(sorted, src, e, xl, xr, n, k, lane);
 }
 
 // Whether sorted[i] equals a neighbour of the sorted array (length n), by order key.
@@ -1320,35 +1401,45 @@ __global__ void __launch_bounds__(DT) decide_kernel(b3_chain_args a) {
     // steady steps read the slots
     bool has = false;
     if (nf == 0) {
-      // score = unbiased variance of normalize(v)
-      const int j = tid;
-      if (j < l) {
-        const T* vr = v + (long long)j * HD;
-        float ss = 0.f;
-        for (int d = 0; d < HD; d += 8) {
-          float x[8];
-          ld8(vr + d, x);
+      // score = unbiased variance of normalize(v); four threads per token, each with a quarter of
+      // its features in registers (one thread per token, reading the row three times, left 6 of
+      // the 8 wavefronts idle: the step took 31 us at HD = 128, now 21; bound by the ordered sums)
+      constexpr int NQ = HD / 4;
+      for (int j = tid >> 2; j < ((l + 127) & ~127); j += DT / 4) {
+        float x[NQ];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
-        }
-        const float nrm = fmaxf(sqrtf(ss), 1e-12f);
-        float mean = 0.f;
-        for (int d = 0; d < HD; d += 8) {
-          float x[8];
-          ld8(vr + d, x);
+        for (int d = 0; d < NQ; d += 8) {
+          if (j < l) ld8(v + (long long)j * HD + (tid & 3) * NQ + d, x + d);
+          else {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) mean += div_rn(x[i], nrm);
+            for (int i = 0; i < 8; ++i) x[d + i] = 0.f;
+          }
         }
-        mean /= (float)HD;
-        float var = 0.f;
-        for (int d = 0; d < HD; d += 8) {
-          float x[8];
-          ld8(vr + d, x);
+        // every sum runs through the row's features in order, from one thread of the four to the
+        // next (the scores order the slots, and the order among equal keep values follows them)
+        auto chain = [&](auto&& add) {
+          float s = 0.f;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) { const float u = div_rn(x[i], nrm) - mean; var += u * u; }
+          for (int q = 0; q < 4; ++q) {
+            float t = q == 0 ? 0.f : __shfl(s, (lane & ~3) + q - 1, 64);
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) add(t, x[i]);
+            s = t;
+          }
+          return __shfl(s, lane | 3, 64);
+        };
+        const float nrm = fmaxf(sqrtf(chain([](float& t, float u) { t += u * u; })), 1e-12f);
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) x[i] = div_rn(x[i], nrm);
+        const float mean = chain([](float& t, float u) { t += u; }) / (float)HD;
+        const float var = chain([&](float& t, float u) {
+          const float c = u - mean;
+          t += c * c;
+        });
+        if (j < l && (tid & 3) == 0) {
+          sm.score[j] = var / (float)(HD - 1);
+          sm.rel[j] = 0.15f;
         }
-        sm.score[j] = var / (float)(HD - 1);
-        sm.rel[j] = 0.15f;
       }
     } else {
       if constexpr (BF) has = score_phase16<HD>(sm, td, td_ready, kr, kp, v, l, steady, scale, wave, lane, log);
@@ -1385,9 +1476,7 @@ __global__ void __launch_bounds__(DT) decide_kernel(b3_chain_args a) {
       sync_lds();
       if (sm.tie) {
         if (wave == 0) {
-          for (int j = lane; j < l; j += WAVE)
-            sm.u.to.e[0][j] = ((uint64_t)tie_key(sm.score[j], true) << 32) | (uint32_t)j;
-          const int fl = tie_order_wave(sm.u.to.e[0], sm.u.to.pr[0], sm.u.to.stk[0], l, m, sm.si_a, lane);
+          const int fl = tie_order(sm.sk_a, sm.si_a, sm.u.to.e[0], sm.u.to.xl[0], sm.u.to.xr[0], l, m, lane);
           if (fl && lane == 0) atomicOr(&sm.tie, B3_TIE_LIMIT);
         }
         sync_lds();
@@ -1652,14 +1741,10 @@ __global__ void __launch_bounds__(DT) decide_kernel(b3_chain_args a) {
       if (const int tie = sm.tie) {
         int fl = 0;
         if (wave == 0 && (tie & B3_TIE_TOP)) {
-          for (int j = lane; j < l; j += WAVE)
-            sm.u.to.e[0][j] = ((uint64_t)tie_key(cand_value(sm, j), true) << 32) | (uint32_t)j;
-          fl = tie_order_wave(sm.u.to.e[0], sm.u.to.pr[0], sm.u.to.stk[0], l, kc, sm.si_a, lane);
+          fl = tie_order(sm.sk_a, sm.si_a, sm.u.to.e[0], sm.u.to.xl[0], sm.u.to.xr[0], l, kc, lane);
         }
         if (wave == 1 && (tie & B3_TIE_BOT)) {
-          for (int j = lane; j < S; j += WAVE)
-            sm.u.to.e[1][j] = ((uint64_t)tie_key(sm.keep[j], false) << 32) | (uint32_t)j;
-          fl = tie_order_wave(sm.u.to.e[1], sm.u.to.pr[1], sm.u.to.stk[1], S, kc, sm.si_b, lane);
+          fl = tie_order(sm.sk_b, sm.si_b, sm.u.to.e[1], sm.u.to.xl[1], sm.u.to.xr[1], S, kc, lane);
         }
         if (fl && lane == 0) atomicOr(&sm.tie, B3_TIE_LIMIT);
         sync_lds();
