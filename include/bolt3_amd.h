@@ -429,10 +429,9 @@ int64_t bolt3_decode_workspace_bytes(int32_t B, int32_t H, int32_t HKV, int32_t 
 /*
  * A whole one-token decode layer step in bf16: the packed input projection
  * x . W_in^T + b_in (W_in rows q | k | v | beta | eta, zero rows padding to n_in), the
- * bolt3_decode step on that row, then out = y . W_out^T + b_out.  The projections stream
- * each weight once (workgroups of 128 weight rows x 512 columns of K, x staged in LDS) and
- * leave fp32 partial products per K chunk in proj_work, added in order and rounded once by
- * their consumer.
+ * bolt3_decode step on that row, then out = y . W_out^T + b_out (rounded, then + res where res
+ * is set).  The projections stream each weight once; the projected rows (B <= 16) or the fp32
+ * partial products of 512-column chunks (B > 16) go through proj_work.
  * Replaces vsa_lm/config/bolt3.py:346-402 for t_s == 1 together with the q/k/v/beta/eta
  * projections it calls (:59-66, :349) and o_proj (:400-402).
  */
@@ -452,10 +451,35 @@ typedef struct {
   int64_t out_row_stride;     /* multiple of 4 */
   float* proj_work;           /* >= bolt3_decode_layer_workspace_bytes(B, d_model, n_in, H*HD, n_out) bytes */
   int64_t proj_work_bytes;
+  const void* res;            /* [B][res_row_stride] added to the rounded output, or NULL; may be out */
+  int64_t res_row_stride;     /* multiple of 4 */
 } b3_decode_layer_args;
 int bolt3_decode_layer(const b3_decode_layer_args* a, void* stream);
-/* Workspace of bolt3_decode_layer's projections (besides dec.work): the fp32 partial products. */
+/* Workspace of bolt3_decode_layer's projections (besides dec.work). */
 int64_t bolt3_decode_layer_workspace_bytes(int32_t B, int32_t d_model, int32_t n_in, int32_t hd_total, int32_t n_out);
+
+/*
+ * A bf16 linear layer on a few rows (one-token decode steps), W read once:
+ *   B3_ROWS_PLAIN     out = round(x . W^T + bias)
+ *   B3_ROWS_SWIGLU    out = round(round(silu(round(x . W^T + bias))) * round(x . W2^T)): gate and up projection of
+ *                     the SwiGLU MLP (vsa_lm/surgery.py:210-211)
+ *   B3_ROWS_RESIDUAL  out = round(round(x . W^T + bias) + res): down or output projection and the residual add
+ * At most 16 rows, N a multiple of 16, K of 32; out may be res.
+ */
+enum { B3_ROWS_PLAIN = 0, B3_ROWS_SWIGLU = 1, B3_ROWS_RESIDUAL = 2 };
+typedef struct {
+  int32_t mode, M, N, K;
+  const void* x;              /* [M][x_row_stride] bf16, 16-byte aligned rows */
+  int64_t x_row_stride;
+  const void* w;              /* [N][K] bf16 */
+  const void* w2;             /* [N][K] bf16, B3_ROWS_SWIGLU only */
+  const void* bias;           /* [N] bf16 or NULL */
+  const void* res;            /* [M][res_row_stride] bf16, B3_ROWS_RESIDUAL only */
+  int64_t res_row_stride;
+  void* out;                  /* [M][out_row_stride] bf16 */
+  int64_t out_row_stride;
+} b3_rows_linear_args;
+int bolt3_rows_linear(const b3_rows_linear_args* a, void* stream);
 
 /*
  * RMSNorm of rows: y = (x * rsqrt(mean(x^2) + eps)) * w with an fp32 statistic, each product

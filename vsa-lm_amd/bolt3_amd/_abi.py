@@ -98,7 +98,7 @@ class DecodeLayerArgs(C.Structure):
     _fields_ = [
         ("dec", DecodeArgs), ("x", p), ("x_row_stride", i64), ("d_model", i32),
         ("w_in", p), ("b_in", p), ("n_in", i32), ("w_out", p), ("b_out", p), ("n_out", i32),
-        ("out", p), ("out_row_stride", i64), ("proj_work", p), ("proj_work_bytes", i64),
+        ("out", p), ("out_row_stride", i64), ("proj_work", p), ("proj_work_bytes", i64), ("res", p), ("res_row_stride", i64),
     ]
 
 
@@ -127,6 +127,14 @@ class AttnBwdArgs(C.Structure):
         ("d_slot_k", p), ("d_slot_v", p), ("d_sink_k", p), ("d_sink_v", p), ("part", i32),
         ("rd_rows", p),
     ]
+
+
+ROWS_PLAIN, ROWS_SWIGLU, ROWS_RESIDUAL = 0, 1, 2   # b3_rows_linear_args.mode
+
+
+class RowsLinearArgs(C.Structure):
+    _fields_ = [("mode", i32), ("M", i32), ("N", i32), ("K", i32), ("x", p), ("x_row_stride", i64), ("w", p),
+                ("w2", p), ("bias", p), ("res", p), ("res_row_stride", i64), ("out", p), ("out_row_stride", i64)]
 
 
 class RmsNormArgs(C.Structure):
@@ -166,7 +174,7 @@ EXPORTS = ("bolt3_attn_bwd", "bolt3_heads", "bolt3_heads_bwd", "bolt3_heads_bwd_
            "bolt3_chain_noalloc", "bolt3_chain_workspace_bytes", "bolt3_chunk_attn",
            "bolt3_decode",
            "bolt3_decode_layer", "bolt3_decode_layer_workspace_bytes", "bolt3_decode_workspace_bytes",
-           "bolt3_rms_norm", "bolt3_slot_keys", "bolt3_step_advance", "bolt3_version", "bolt3_wait_count")
+           "bolt3_rms_norm", "bolt3_rows_linear", "bolt3_slot_keys", "bolt3_step_advance", "bolt3_version", "bolt3_wait_count")
 
 _lib = None
 
@@ -184,7 +192,7 @@ def load():
                      ("bolt3_chunk_attn", AttnArgs),
                      ("bolt3_decode", DecodeArgs), ("bolt3_decode_layer", DecodeLayerArgs),
                      ("bolt3_slot_keys", SlotKeysArgs), ("bolt3_attn_bwd", AttnBwdArgs),
-                     ("bolt3_rms_norm", RmsNormArgs), ("bolt3_chain_bwd", ChainBwdArgs),
+                     ("bolt3_rms_norm", RmsNormArgs), ("bolt3_rows_linear", RowsLinearArgs), ("bolt3_chain_bwd", ChainBwdArgs),
                      ("bolt3_heads_bwd", HeadsBwdArgs)):
         fn = getattr(lib, name)
         fn.argtypes = [C.POINTER(st), p]

@@ -29,6 +29,7 @@ import torch.nn.functional as F
 
 from . import _abi as A
 from .bolt3 import N_SINKS, Bolt3Attn, _check_dtype, _gout, _tout
+from .layers import mlp_rows
 
 DONE_CHECK_EVERY = 16      # tokens between the all-rows-done tests (the reference's period)
 
@@ -57,6 +58,15 @@ def _fused_step_ok(dt: torch.dtype, d_model: int, hd_total: int, n_out: int) -> 
     a multiple of 16, and at most 8 K chunks of 512 in either projection."""
     return dt == torch.bfloat16 and d_model >= 32 and d_model % 32 == 0 and n_out % 16 == 0 and \
         (d_model + 511) // 512 <= 8 and (hd_total + 511) // 512 <= 8
+
+
+def _set_residual(la, res: torch.Tensor | None, B: int, n_out: int, dt: torch.dtype) -> bool:
+    """Hand the residual rows to the fused layer step (its output then is res + layer); False where
+    their dtype, shape or layout is not one it takes (the caller adds them)."""
+    ok = res is not None and res.dtype == dt and res.numel() == B * n_out and res.shape[-1] == n_out and \
+        res.is_contiguous() and res.data_ptr() % 8 == 0 and n_out % 4 == 0
+    la.res, la.res_row_stride = (res.data_ptr(), n_out) if ok else (None, 0)
+    return ok
 
 
 class AnchorCache:
@@ -449,8 +459,8 @@ class Bolt3Decoder:
     # ------------------------------------------------------------ one Bolt-3 layer
 
     def _bolt3_layer(self, ly: Bolt3Attn, h, pos_start: int, m_state: torch.Tensor, st: Bolt3LayerState,
-                     record=None, desc: int | None = None):
-        """One step of a Bolt-3 layer on t tokens.  ``desc``: device address of a step descriptor
+                     record=None, desc: int | None = None, res: torch.Tensor | None = None):
+        """One step of a Bolt-3 layer on t tokens (``res``: plus these rows).  ``desc``: device address of a step descriptor
         (graph capture): the fused one-token kernels then take the position and ring segments from
         it, and the ring bookkeeping and consolidation are left to the caller."""
         B, t, _ = h.shape
@@ -510,8 +520,11 @@ class Bolt3Decoder:
                 out = torch.empty(B, 1, side["wo"].shape[0], dtype=dt, device=dev)
                 call_args.x, call_args.out = h.data_ptr(), out.data_ptr()
                 a.step_desc, a.ring_cap = desc, st.cap
+                added = _set_residual(call_args, res, B, out.shape[-1], dt)
                 A.call("bolt3_decode_layer", call_args, dev)
                 a.step_desc = None
+                if res is not None and not added:
+                    out = res + out
                 if desc is None:
                     st.cur = (cs, cl + 1)
                     if st.cur[1] >= ly.C:
@@ -553,7 +566,7 @@ class Bolt3Decoder:
         out = F.linear(y, side["wo"])
         if st.cur[1] >= ly.C:
             self._consolidate(ly, st, m_state, gam, side, record)
-        return out
+        return out if res is None else res + out
 
     def _bolt3_prefill(self, ly: Bolt3Attn, h: torch.Tensor, m_state: torch.Tensor, st: Bolt3LayerState,
                        record=None):
@@ -680,7 +693,8 @@ class Bolt3Decoder:
             self._scratch_bufs[(dev, name)] = t
         return t
 
-    def _anchor_fused(self, ly, h: torch.Tensor, pos_start: int, cache: AnchorCache, desc: int | None = None):
+    def _anchor_fused(self, ly, h: torch.Tensor, pos_start: int, cache: AnchorCache, desc: int | None = None,
+                      res: torch.Tensor | None = None):
         """One token of a softmax-anchor layer as one bolt3_decode_layer call in its anchor mode:
         q | k | v projection, q/k norm and RoPE, the new key and value appended to the cache,
         causal softmax over the cache, o_proj.  ``desc`` as in _bolt3_layer (cache.n is then the
@@ -715,19 +729,21 @@ class Bolt3Decoder:
         la.w_out, la.b_out, la.n_out, la.out_row_stride = side["wo"].data_ptr(), None, n_out, n_out
         out = torch.empty(B, 1, n_out, dtype=dt, device=dev)
         la.out = out.data_ptr()
+        added = _set_residual(la, res, B, n_out, dt)
         A.call("bolt3_decode_layer", la, dev)
         if desc is None:
             cache.n += 1
-        return out
+        return res + out if res is not None and not added else out
 
-    def _anchor_layer(self, ly, h: torch.Tensor, pos_start: int, cache: AnchorCache) -> torch.Tensor:
+    def _anchor_layer(self, ly, h: torch.Tensor, pos_start: int, cache: AnchorCache,
+                      res: torch.Tensor | None = None) -> torch.Tensor:
         """Causal softmax attention of t new tokens over the cached ones and themselves
         (vsa_lm/config/bolt3.py:426-445): query i sees cached keys and new keys up to i.  One bf16
         token: the fused HIP step; otherwise torch's attention on the cache."""
         b, t, _ = h.shape
         if t == 1 and self.fuse_projections and _fused_step_ok(h.dtype, h.shape[-1], ly.H * ly.HD,
                                                                ly.o_proj.out_features) and ly.G <= 8:
-            return self._anchor_fused(ly, h, pos_start, cache)
+            return self._anchor_fused(ly, h, pos_start, cache, res=res)
         q, k, v = ly.head_qkv(h)
         q, k = ly.rope(q, pos_start=pos_start), ly.rope(k, pos_start=pos_start)
         n_old = cache.n
@@ -742,7 +758,15 @@ class Bolt3Decoder:
                 visible = torch.ones(t, n_old + t, dtype=torch.bool, device=h.device).tril(diagonal=n_old)
             y = F.scaled_dot_product_attention(q, keys.to(q.dtype), vals.to(q.dtype), attn_mask=visible,
                                                enable_gqa=ly.G > 1)
-        return ly.o_proj(y.transpose(1, 2).reshape(b, t, ly.H * ly.HD))
+        out = ly.o_proj(y.transpose(1, 2).reshape(b, t, ly.H * ly.HD))
+        return out if res is None else res + out
+
+    @staticmethod
+    def _mlp(blk, x: torch.Tensor) -> torch.Tensor:
+        """x + MLP(norm2(x)); the few rows of a one-token step stream the weights in two launches."""
+        h = blk.norm2(x)
+        y = mlp_rows(blk.mlp, h, x)
+        return x + blk.mlp(h) if y is None else y
 
     # ------------------------------------------------------------ model-level API
 
@@ -765,10 +789,10 @@ class Bolt3Decoder:
                 h = blk.norm1(x)
                 if hasattr(blk, "vsa"):
                     rec = record.setdefault(li, []) if isinstance(record, dict) else record
-                    x = x + self._bolt3_layer(blk.vsa, h, pos_start, states[li], kv_caches[li], rec)
+                    x = self._bolt3_layer(blk.vsa, h, pos_start, states[li], kv_caches[li], rec, res=x)
                 else:
-                    x = x + self._anchor_layer(blk.attn, h, pos_start, kv_caches[li])
-                x = x + blk.mlp(blk.norm2(x))
+                    x = self._anchor_layer(blk.attn, h, pos_start, kv_caches[li], res=x)
+                x = self._mlp(blk, x)
             return m.norm(x), states, kv_caches
 
     def _feed(self, ids: torch.Tensor, pos: int, states, kv_caches):
@@ -959,11 +983,10 @@ class DecodeGraph:
         for li, blk in enumerate(m.blocks):
             h = blk.norm1(x)
             if hasattr(blk, "vsa"):
-                y = dec._bolt3_layer(blk.vsa, h, self.pos, self.states[li], self.kv[li], desc=d_b3)
+                x = dec._bolt3_layer(blk.vsa, h, self.pos, self.states[li], self.kv[li], desc=d_b3, res=x)
             else:
-                y = dec._anchor_fused(blk.attn, h, self.pos, self.kv[li], desc=d_an)
-            x = x + y
-            x = x + blk.mlp(blk.norm2(x))
+                x = dec._anchor_fused(blk.attn, h, self.pos, self.kv[li], desc=d_an, res=x)
+            x = dec._mlp(blk, x)
         return m.lm_head(m.norm(x)[:, -1])
 
     def _write_descriptors(self):

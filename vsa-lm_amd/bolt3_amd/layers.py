@@ -6,7 +6,8 @@ unchanged.  ``SoftmaxAttn``, ``MLP`` and ``HybridLM`` are the caller side of the
 path (the softmax-anchor layers and the model container that
 ``Bolt3Decoder`` walks); they run as PyTorch ops on the device, except
 ``RMSNorm``, whose device forward is the library's ``bolt3_rms_norm`` (one pass
-per row instead of the torch ops' six; CPU tensors keep the torch ops).
+per row instead of the torch ops' six; CPU tensors keep the torch ops), and the
+MLP of a one-token decode step (``mlp_rows``).
   RMSNorm      -- vsa_lm/surgery.py:43-53
   rope_inv_freq-- vsa_lm/surgery.py:56-72
   RoPE         -- vsa_lm/surgery.py:80-93
@@ -101,6 +102,55 @@ class MLP(nn.Module):
 
     def forward(self, x):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+
+
+MLP_ROWS = 16   # rows bolt3_rows_linear takes; the library's products are the faster ones above
+
+
+def _plain_linear(m: nn.Module, x: torch.Tensor) -> bool:
+    """A linear layer that is nothing but its bf16 weight on x's device, rows as the kernel reads them."""
+    return (type(m) is nn.Linear and m.bias is None and not m._forward_hooks and not m._forward_pre_hooks and
+            type(m.weight) in (nn.Parameter, torch.Tensor) and m.weight.dtype == torch.bfloat16 and
+            m.weight.device == x.device and m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0 and
+            m.in_features % 32 == 0 and m.out_features % 16 == 0)
+
+
+def mlp_rows(mlp: nn.Module, h: torch.Tensor, res: torch.Tensor) -> torch.Tensor | None:
+    """res + mlp(h) for the few rows of a one-token decode step, in two launches that stream the weights
+    once (gate, up and SwiGLU; down and the residual), with the roundings of the module's own ops.
+    None where it does not apply: gradients, autocast or hooks, other modules, dtypes or layouts,
+    more than MLP_ROWS rows."""
+    D = h.shape[-1]
+    M = h.numel() // D if D else 0
+    if (type(mlp) is not MLP or not 0 < M <= MLP_ROWS or not h.is_cuda or h.dtype != torch.bfloat16 or
+            res.dtype != h.dtype or res.shape != h.shape or res.device != h.device or
+            type(h) is not torch.Tensor or type(res) is not torch.Tensor or torch.is_grad_enabled() or
+            torch.is_autocast_enabled(h.device.type) or mlp._forward_hooks or mlp._forward_pre_hooks or
+            torch.nn.modules.module._has_any_global_hook()):
+        return None
+    gate, up, down = mlp.gate_proj, mlp.up_proj, mlp.down_proj
+    if not (_plain_linear(gate, h) and _plain_linear(up, h) and _plain_linear(down, h)):
+        return None
+    inner = gate.out_features
+    if gate.in_features != D or up.in_features != D or up.out_features != inner or \
+            down.in_features != inner or down.out_features != D:
+        return None
+    from . import _abi as A
+    x, r = h.reshape(M, D), res.reshape(M, D)
+    x = x if x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 else x.contiguous()
+    r = r if r.stride(1) == 1 and r.stride(0) % 4 == 0 and r.data_ptr() % 8 == 0 else r.contiguous()
+    act = torch.empty(M, inner, dtype=h.dtype, device=h.device)
+    out = torch.empty(M, D, dtype=h.dtype, device=h.device)
+    a = A.RowsLinearArgs()
+    a.mode, a.M, a.N, a.K = A.ROWS_SWIGLU, M, inner, D
+    a.x, a.x_row_stride, a.w, a.w2 = x.data_ptr(), x.stride(0), gate.weight.data_ptr(), up.weight.data_ptr()
+    a.out, a.out_row_stride = act.data_ptr(), inner
+    A.call("bolt3_rows_linear", a, h.device)
+    a.mode, a.N, a.K = A.ROWS_RESIDUAL, D, inner
+    a.x, a.x_row_stride, a.w, a.w2 = act.data_ptr(), inner, down.weight.data_ptr(), None
+    a.res, a.res_row_stride, a.out, a.out_row_stride = r.data_ptr(), r.stride(0), out.data_ptr(), D
+    A.call("bolt3_rows_linear", a, h.device)
+    return out.view(h.shape)
 
 
 class SoftmaxAttn(nn.Module):

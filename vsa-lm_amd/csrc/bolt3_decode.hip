@@ -13,13 +13,16 @@
 //   fp32: decode_split_kernel, grid (ceil(keys / 128) + HD/32, B*HKV), 128-key pieces and
 //     32-row readout pieces in parallel with fp32 MFMAs, then decode_combine_kernel, grid
 //     (B*HKV), merges the partial softmaxes and finishes the readout.
-// bolt3_decode_layer (bf16) adds the two projections around these: rowproj_kernel streams
-// a weight once per step and leaves fp32 partial products per K chunk; the prep kernel sums
-// those of the input projection and proj_reduce_kernel those of o_proj.
+// bolt3_decode_layer (bf16) adds the two projections around these: up to 16 rows in one kernel
+// each (bolt3_rows.h); above, rowproj_kernel streams a weight once per step and leaves fp32
+// partial products per K chunk; the prep kernel sums those of the input projection and
+// proj_reduce_kernel those of o_proj.
+#include <algorithm>
 #include <utility>
 
 #include "bolt3_common.h"
 #include "bolt3_math.h"
+#include "bolt3_rows.h"
 #include "bolt3_amd.h"
 
 namespace b3 {
@@ -1071,9 +1074,10 @@ __global__ void __launch_bounds__(64 * NW, 2) rowproj_kernel(ProjArgs p) {
   }
 }
 
-// y[m][n] = round(sum over chunks of parts + bias), four n per thread
+// y[m][n] = round(sum over chunks of parts + bias), + res[m][n] where res is set; four n per thread
 __global__ void __launch_bounds__(256) proj_reduce_kernel(const float* parts, int n_chunks, int M, int N,
-                                                          const uint16_t* bias, uint16_t* y, int64_t y_rs) {
+                                                          const uint16_t* bias, const uint16_t* res, int64_t res_rs,
+                                                          uint16_t* y, int64_t y_rs) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   const int m = i / (N / 4), n = 4 * (i % (N / 4));
   if (m >= M) return;
@@ -1088,6 +1092,11 @@ __global__ void __launch_bounds__(256) proj_reduce_kernel(const float* parts, in
   u16x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = f2bf(bias ? v[e] + bf2f(bias[n + e]) : v[e]);
+  if (res) {
+    const u16x4 r = *reinterpret_cast<const u16x4*>(res + (long long)m * res_rs + n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = f2bf(add_rn(bf2f(o[e]), bf2f(r[e])));
+  }
   *reinterpret_cast<u16x4*>(y + (long long)m * y_rs + n) = o;
 }
 
@@ -1182,6 +1191,7 @@ extern "C" int bolt3_decode(const b3_decode_args* a, void* stream) {
 extern "C" int64_t bolt3_decode_layer_workspace_bytes(int32_t B, int32_t d_model, int32_t n_in, int32_t hd_total,
                                                       int32_t n_out) {
   if (B <= 0 || d_model <= 0 || n_in <= 0 || hd_total <= 0 || n_out <= 0) return 0;
+  if (B <= b3::ROWS_MAX) return ((int64_t)B * n_in * 2 + 15) / 16 * 16;   // the projected rows, rounded
   const long long a = b3::proj_parts_floats(B, n_in, d_model), b = b3::proj_parts_floats(B, n_out, hd_total);
   return (int64_t)(a > b ? a : b) * 4;
 }
@@ -1202,9 +1212,29 @@ extern "C" int bolt3_decode_layer(const b3_decode_layer_args* a, void* stream) {
       reinterpret_cast<uintptr_t>(a->proj_work) % 16)
     return B3_ERR_ARG;
   if (b3::proj_chunks(a->d_model) > b3::LP_MAXC || b3::proj_chunks(hd_total) > b3::LP_MAXC) return B3_ERR_UNSUPPORTED;
+  if (a->res && (a->res_row_stride < a->n_out || a->res_row_stride % 4 || reinterpret_cast<uintptr_t>(a->res) % 8))
+    return B3_ERR_ARG;
   if (a->proj_work_bytes < bolt3_decode_layer_workspace_bytes(d.B, a->d_model, a->n_in, hd_total, a->n_out))
     return B3_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  using u16 = const uint16_t*;
+  if (d.B <= b3::ROWS_MAX) {
+    b3_decode_args step = d;
+    step.lin = a->proj_work;
+    const b3::RowsArgs pin{static_cast<u16>(a->x), a->x_row_stride, static_cast<u16>(a->w_in), nullptr,
+                           static_cast<u16>(a->b_in), nullptr, 0, reinterpret_cast<uint16_t*>(a->proj_work), a->n_in,
+                           d.B, a->n_in, a->d_model};
+    rc = b3::launch_rows<b3::ROWS_PLAIN>(pin, st);
+    if (rc) return rc;
+    const b3::LinParts none{nullptr, 0, 0, nullptr};
+    rc = d.HD == 64 ? b3::launch_decode<uint16_t, 64>(step, st, none)
+                    : b3::launch_decode<uint16_t, 128>(step, st, none);
+    if (rc) return rc;
+    const b3::RowsArgs pout{static_cast<u16>(d.y), hd_total, static_cast<u16>(a->w_out), nullptr,
+                            static_cast<u16>(a->b_out), static_cast<u16>(a->res), a->res_row_stride,
+                            static_cast<uint16_t*>(a->out), a->out_row_stride, d.B, a->n_out, hd_total};
+    return a->res ? b3::launch_rows<b3::ROWS_RESIDUAL>(pout, st) : b3::launch_rows<b3::ROWS_PLAIN>(pout, st);
+  }
   const b3::ProjArgs pin{reinterpret_cast<const uint16_t*>(a->x), a->x_row_stride,
                          reinterpret_cast<const uint16_t*>(a->w_in), a->proj_work, d.B, a->n_in, a->d_model};
   rc = b3::launch_rowproj(pin, st);
@@ -1219,8 +1249,8 @@ extern "C" int bolt3_decode_layer(const b3_decode_layer_args* a, void* stream) {
   if (rc) return rc;
   const int n_thr = d.B * (a->n_out / 4);
   hipLaunchKernelGGL(b3::proj_reduce_kernel, dim3((n_thr + 255) / 256), dim3(256), 0, st, a->proj_work,
-                     b3::proj_chunks(hd_total), d.B, a->n_out, reinterpret_cast<const uint16_t*>(a->b_out),
-                     reinterpret_cast<uint16_t*>(a->out), a->out_row_stride);
+                     b3::proj_chunks(hd_total), d.B, a->n_out, static_cast<u16>(a->b_out), static_cast<u16>(a->res),
+                     a->res_row_stride, static_cast<uint16_t*>(a->out), a->out_row_stride);
   return (int)hipGetLastError();
 }
 
