@@ -34,6 +34,22 @@ def test_rms_norm_matches_torch(dt, wdt, shape, gpu):
     assert bool((d <= tol).all()), float((d / tol).max())
 
 
+@pytest.mark.parametrize("rows,dim", [(1, 520), (3, 512), (256, 2560), (257, 2560), (2, 8192), (2, 8200)])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_rms_norm_row_and_wave_kernels(rows, dim, offset, gpu):
+    """Both sides of the rule that gives every row a workgroup, and a weight that is not 16-byte aligned."""
+    from bolt3_amd import RMSNorm
+    g = torch.Generator(device=gpu).manual_seed(rows + dim)
+    x = torch.randn(rows, dim, generator=g, device=gpu).to(torch.bfloat16)
+    norm = RMSNorm(dim, 1e-6).to(gpu)
+    w = (torch.rand(dim + offset, generator=g, device=gpu) + 0.5).to(torch.bfloat16)[offset:]
+    norm.weight.data = w
+    with torch.no_grad():
+        y, ref = norm(x), _torch_rms(x, w, 1e-6)
+    d = (y.float() - ref.float()).abs()
+    assert bool((d <= ref.float().abs() * 2 ** -7 + 1e-30).all())
+
+
 def test_rms_norm_strided_rows_and_cpu(gpu):
     from bolt3_amd import RMSNorm
     norm = RMSNorm(128, 1e-5).to(gpu)

@@ -39,11 +39,67 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(b3_rms_norm_args a) {
   }
 }
 
+// Few rows: one workgroup per row, the row in registers (NV pieces of 8 elements per thread), so that
+// the row is read once and by four wavefronts.  One row of 2560 in bf16, latency bound: 4.1 us a
+// launch in a captured decode step against 5.9 for the kernel above, where one wavefront reads
+// the row twice.
+constexpr int RN_NT = 256, RN_NV = 4;
+
+template <typename T, typename W>
+__global__ void __launch_bounds__(RN_NT) rms_norm_row_kernel(b3_rms_norm_args a) {
+  __shared__ float part[RN_NT / 64];
+  const int tid = threadIdx.x, n8 = a.dim / 8;
+  const T* x = reinterpret_cast<const T*>(a.x) + (long long)blockIdx.x * a.x_row_stride;
+  T* y = reinterpret_cast<T*>(a.y) + (long long)blockIdx.x * a.y_row_stride;
+  Vec8<T> v[RN_NV];
+  Vec8<W> w[RN_NV];
+#pragma unroll
+  for (int q = 0; q < RN_NV; ++q)
+    if (tid + RN_NT * q < n8) {
+      v[q].load(x + 8 * (tid + RN_NT * q));
+      w[q].load(reinterpret_cast<const W*>(a.w) + 8 * (tid + RN_NT * q));
+    }
+  float ss = 0.f;
+#pragma unroll
+  for (int q = 0; q < RN_NV; ++q)
+    if (tid + RN_NT * q < n8)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float f = v[q].get(e);
+        ss += f * f;
+      }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) part[tid >> 6] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < RN_NT / 64; ++i) ss += part[i];
+  const float r = 1.0f / sqrtf(div_rn(ss, (float)a.dim) + a.eps);
+#pragma unroll
+  for (int q = 0; q < RN_NV; ++q)
+    if (tid + RN_NT * q < n8) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[q].set(e, mul_rn(mul_rn(v[q].get(e), r), w[q].get(e)));
+      v[q].store(y + 8 * (tid + RN_NT * q));
+    }
+}
+
+// One workgroup per row up to a row per compute unit, where every row's latency shows, if the row fits
+// the registers, is long enough for four wavefronts and its weight may be read in 16-byte pieces.
+constexpr int RN_MAX_ROWS = 256;
+
+template <typename T, typename W>
+static void launch_rms_w(const b3_rms_norm_args& a, hipStream_t st) {
+  if (a.rows <= RN_MAX_ROWS && a.dim > 8 * 64 && a.dim <= 8 * RN_NT * RN_NV && reinterpret_cast<uintptr_t>(a.w) % 16 == 0)
+    hipLaunchKernelGGL((rms_norm_row_kernel<T, W>), dim3((unsigned)a.rows), dim3(RN_NT), 0, st, a);
+  else
+    hipLaunchKernelGGL((rms_norm_kernel<T, W>), dim3((unsigned)((a.rows + 3) / 4)), dim3(256), 0, st, a);
+}
+
 template <typename T>
 static int launch_rms(const b3_rms_norm_args& a, hipStream_t st) {
-  const dim3 grid((unsigned)((a.rows + 3) / 4));
-  if (a.w_dtype == B3_F32) hipLaunchKernelGGL((rms_norm_kernel<T, float>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((rms_norm_kernel<T, uint16_t>), grid, dim3(256), 0, st, a);
+  if (a.w_dtype == B3_F32) launch_rms_w<T, float>(a, st);
+  else launch_rms_w<T, uint16_t>(a, st);
   return (int)hipGetLastError();
 }
 
