@@ -69,3 +69,27 @@ def test_forward_counts_first_group_and_wait_changes_nothing(gpu):
         torch.cuda.synchronize()
         assert int(ctr[0].item()) - before == 2 * CFG["num_kv_heads"]
     assert torch.equal(y_gated, y_plain)
+
+
+@pytest.mark.parametrize("B,T", [(1, 385), (2, 1600), (2, 1700), (1, 2944), (1, 2945)])
+def test_group_count_changes_no_decision(B, T, gpu):
+    """One, two and three step groups (the rule's edges: 2, 11, 12, 21 and 22 steps): the same attention, so
+    outputs that differ by o_proj's rounding at most (its products have other row counts)."""
+    from bolt3_amd import Bolt3Attn
+    from bolt3_amd import bolt3 as B3
+    import recipes
+    print(f"[case] step groups B={B} T={T}", flush=True)
+    torch.manual_seed(1)
+    mod = recipes.init_module(Bolt3Attn(CFG), 5, nondefault=True).to(torch.bfloat16).to(gpu)
+    x = torch.randn(B, T, CFG["dim"], device=gpu).to(torch.bfloat16)
+    rule, ys = B3._n_groups, []
+    try:
+        with torch.no_grad():
+            ys.append(mod(x).float())
+            for k in (1, 2, 3):
+                B3._n_groups = lambda n, k=k: k
+                ys.append(mod(x).float())
+    finally:
+        B3._n_groups = rule
+    for y in ys[1:]:   # one rounding of each element and fp32 sums of 512 products
+        assert bool(((y - ys[0]).abs() <= 2.0 ** -7 * ys[0].abs() + 1e-4 * ys[0].abs().max()).all())

@@ -42,6 +42,10 @@ def test_step_groups_of_the_benchmark_forward():
     assert len(g) == 16 and max(s1 - s0 for s0, s1 in g) <= 33
 
 
+def test_short_sequences_take_fewer_groups():
+    assert [_n_groups(n) for n in (1, 11, 12, 21, 22, 111, 112)] == [1, 1, 2, 2, 3, 3, 4]
+
+
 def test_packed_parameters_follow_in_place_updates():
     torch.manual_seed(0)
     mod = Bolt3Attn(CFG)

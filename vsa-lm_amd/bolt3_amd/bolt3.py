@@ -71,6 +71,13 @@ def _wait_started(dev: torch.device, counter: torch.Tensor, target: int) -> None
 # The forward's consolidation steps are issued in this many groups, so that the slot field and
 # readout of early chunks run while the chain still decides later steps.
 CHAIN_GROUPS = 3
+# A group costs the host about 85 us (three chain launches on two streams, the attention, o_proj),
+# and a step about 17 us of chain: short sequences, whose forward is bound by the host's launches,
+# take fewer.  Forward of a Qwen3-4B-shape layer with 1 / 2 / 3 groups, us: 5 steps (1 x 777 tokens)
+# 309 / 403 / 480; 9 steps (1 x 1400) 359 / 435 / 517, (4 x 1400) 570 / 562 / 600; 14 steps (1 x 2000)
+# 470 / 466 / 563, (4 x 2000) 775 / 704 / 749; 22 steps (1 x 3000) 670 / 620 / 614; 30 steps
+# (4 x 4096) 1594 / 1354 / 1297.
+ONE_GROUP_STEPS, TWO_GROUP_STEPS = 11, 21
 # ... and at least one group per this many steps, so that the work left after the last group's
 # slot decisions (its M_res updates, attention and o_proj) stays short on long sequences
 GROUP_STEPS = 32
@@ -83,6 +90,8 @@ FUSED_Q_PREP = True
 
 
 def _n_groups(n_steps: int) -> int:
+    if n_steps <= TWO_GROUP_STEPS:
+        return 1 if n_steps <= ONE_GROUP_STEPS else 2
     return max(CHAIN_GROUPS, round(n_steps / GROUP_STEPS))
 
 
@@ -362,7 +371,8 @@ class Bolt3Attn(nn.Module):
         first_started = None
         if n_cons > 0:
             s_dec = A.side_stream(dev, 0)
-            s_m = A.side_stream(dev, 1) if split else s_dec
+            two = split and len(groups) > 1   # decisions and M_res updates on streams of their own
+            s_m = A.side_stream(dev, 1) if two else s_dec
             # n_filled = 0: the chain builds the empty state itself, these are outputs only
             st = dict(ak=torch.empty(bh, S, HD, dtype=dt, device=dev), av=torch.empty(bh, S, HD, dtype=dt, device=dev),
                       mass=torch.empty(bh, S, device=dev), util=torch.empty(bh, S, device=dev),
@@ -403,19 +413,16 @@ class Bolt3Attn(nn.Module):
                 if snap_mp is not None:
                     kw.update(snap_mass=snap_mp[0][s0:s1], snap_pm=snap_mp[1][s0:s1])
                 started = None
-                if split:
-                    count = ctr is not None and s0 == 0
-                    with torch.cuda.stream(s_dec):
-                        self._chain(*args, phase=1, started=ctr[0].data_ptr() if count else None, **kw)
-                    if count:
-                        ctr[1] += bh
-                        started = ctr[1]
+                count = ctr is not None and s0 == 0
+                with torch.cuda.stream(s_dec):
+                    self._chain(*args, phase=1 if two else 0, started=ctr[0].data_ptr() if count else None, **kw)
+                if count:
+                    ctr[1] += bh
+                    started = ctr[1]
+                if two:
                     s_m.wait_stream(s_dec)
                     with torch.cuda.stream(s_m):
                         self._chain(*args, phase=2, **kw)
-                else:
-                    with torch.cuda.stream(s_dec):
-                        self._chain(*args, **kw)
                 ev = torch.cuda.Event()
                 ev.record(s_m)
                 done.append(ev)
@@ -471,7 +478,7 @@ class Bolt3Attn(nn.Module):
             spans = [(0, min(T, (groups[0][1] + 2) * C))] + \
                     [(min(T, (s0 + 2) * C), min(T, (s1 + 2) * C)) for s0, s1 in groups[1:]]
             y_all = torch.empty(b * T * K, dtype=dt, device=dev)
-            out = torch.empty(b, T, side["wo"].shape[0], dtype=dt, device=dev)
+            out = torch.empty(b, T, side["wo"].shape[0], dtype=dt, device=dev) if len(groups) > 1 else None
             esz, off = y_all.element_size(), 0
             a.part = 0
             for gi, ((s0, s1), ev) in enumerate(zip(groups, done)):
@@ -484,7 +491,9 @@ class Bolt3Attn(nn.Module):
                 # writes rows t >= t0 only)
                 a.y, a.y_sb, a.y_st = blk.data_ptr() - t0 * K * esz, (t1 - t0) * K, K
                 A.call("bolt3_chunk_attn", a, dev)
-                if b == 1:   # the group's output rows are one contiguous slab of the result
+                if out is None:   # one group: its block is the whole output
+                    out = F.linear(blk, side["wo"]).view(b, T, -1)
+                elif b == 1:   # the group's output rows are one contiguous slab of the result
                     torch.mm(blk, side["wo"].t(), out=out[0, t0:t1])
                 else:
                     out[:, t0:t1].copy_(F.linear(blk, side["wo"]).view(b, t1 - t0, -1))
