@@ -459,6 +459,36 @@ int bolt3_decode_layer(const b3_decode_layer_args* a, void* stream);
 int64_t bolt3_decode_layer_workspace_bytes(int32_t B, int32_t d_model, int32_t n_in, int32_t hd_total, int32_t n_out);
 
 /*
+ * Gradients of the layer's small parameters, each the whole sum of partial sums that the other
+ * backward entry points leave (one launch).  Replaces the reductions autograd makes of
+ * vsa_lm/config/bolt3.py:56-57 (gamma's sigmoid and clamp), :59-66 (biases, norm weights), :238-241
+ * (kappa log(max(mass, 1))) and :253-256 (res_norm).
+ */
+typedef struct {
+  int32_t dtype;              /* of dz */
+  int32_t B, T, H, HKV, HD, S, n_chunks, n_qtiles, n_steps;
+  int32_t n_blocks;           /* rows of d_qn_w / d_kn_w (bolt3_heads_bwd_blocks) */
+  const float* d_res_w;       /* [B*HKV][n_chunks][HD] (bolt3_attn_bwd) */
+  const float* d_gamma;       /* [B*HKV][n_chunks] (bolt3_attn_bwd) */
+  const float* d_bias;        /* [n_steps][B*H][n_qtiles][S] (bolt3_attn_bwd); n_steps > 0 */
+  const float* snap_mass;     /* [n_steps][B*HKV][S] slot mass after every step; n_steps > 0 */
+  const float* d_gamma_chain; /* [n_steps][B*HKV][HD/32] (bolt3_chain_bwd); n_steps > 0 */
+  const float* d_qn_w;        /* [n_blocks][HD] (bolt3_heads_bwd) or NULL */
+  const float* d_kn_w;
+  const void* dz;             /* [B*T][dz_row_stride] the packed projection gradient; n_bias > 0 */
+  int64_t dz_row_stride;
+  int32_t bias_col, n_bias;   /* columns bias_col .. bias_col + n_bias - 1 of dz are summed into g_bias */
+  const float* log_gamma;     /* [HKV] */
+  float* g_res_w;             /* out: [HD] */
+  float* g_qn_w;              /* out: [HD] (d_qn_w) */
+  float* g_kn_w;
+  float* g_bias;              /* out: [n_bias] */
+  float* g_kappa;             /* out: [HKV] */
+  float* g_log_gamma;         /* out: [HKV] */
+} b3_param_grads_args;
+int bolt3_param_grads(const b3_param_grads_args* a, void* stream);
+
+/*
  * A bf16 linear layer on a few rows (one-token decode steps), W read once:
  *   B3_ROWS_PLAIN     out = round(x . W^T + bias)
  *   B3_ROWS_SWIGLU    out = round(round(silu(round(x . W^T + bias))) * round(x . W2^T)): gate and up projection of

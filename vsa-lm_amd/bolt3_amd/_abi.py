@@ -169,11 +169,22 @@ class HeadsBwdArgs(C.Structure):
     ]
 
 
+class ParamGradsArgs(C.Structure):
+    _fields_ = [
+        ("dtype", i32), ("B", i32), ("T", i32), ("H", i32), ("HKV", i32), ("HD", i32), ("S", i32), ("n_chunks", i32),
+        ("n_qtiles", i32), ("n_steps", i32), ("n_blocks", i32),
+        ("d_res_w", p), ("d_gamma", p), ("d_bias", p), ("snap_mass", p), ("d_gamma_chain", p), ("d_qn_w", p),
+        ("d_kn_w", p), ("dz", p), ("dz_row_stride", i64), ("bias_col", i32), ("n_bias", i32), ("log_gamma", p),
+        ("g_res_w", p), ("g_qn_w", p), ("g_kn_w", p), ("g_bias", p), ("g_kappa", p), ("g_log_gamma", p),
+    ]
+
+
 EXPORTS = ("bolt3_attn_bwd", "bolt3_heads", "bolt3_heads_bwd", "bolt3_heads_bwd_blocks", "bolt3_chain",
            "bolt3_chain_bwd", "bolt3_chain_bwd_workspace_bytes",
            "bolt3_chain_noalloc", "bolt3_chain_workspace_bytes", "bolt3_chunk_attn",
            "bolt3_decode",
            "bolt3_decode_layer", "bolt3_decode_layer_workspace_bytes", "bolt3_decode_workspace_bytes",
+           "bolt3_param_grads",
            "bolt3_rms_norm", "bolt3_rows_linear", "bolt3_slot_keys", "bolt3_step_advance", "bolt3_version", "bolt3_wait_count")
 
 _lib = None
@@ -193,7 +204,7 @@ def load():
                      ("bolt3_decode", DecodeArgs), ("bolt3_decode_layer", DecodeLayerArgs),
                      ("bolt3_slot_keys", SlotKeysArgs), ("bolt3_attn_bwd", AttnBwdArgs),
                      ("bolt3_rms_norm", RmsNormArgs), ("bolt3_rows_linear", RowsLinearArgs), ("bolt3_chain_bwd", ChainBwdArgs),
-                     ("bolt3_heads_bwd", HeadsBwdArgs)):
+                     ("bolt3_heads_bwd", HeadsBwdArgs), ("bolt3_param_grads", ParamGradsArgs)):
         fn = getattr(lib, name)
         fn.argtypes = [C.POINTER(st), p]
         fn.restype = C.c_int

@@ -13,8 +13,9 @@ HIP forward keeps, in four C calls and the projections' products:
   token keys and values (:121-155, :182-191), M_res follows the Gershgorin-scaled delta rule
   (:157-166);
 * ``bolt3_heads_bwd``: RoPE, the q/k RMSNorm and the gates' sigmoid / tanh back to the packed
-  projection output; gamma's clamp and the projections close the chain back to x and the
-  parameters.
+  projection output; the projections close the chain back to x and the weights;
+* ``bolt3_param_grads``: the partial sums of the others to the norm weights, kappa, gamma (through
+  its clamp) and the biases.
 
 There is no second path: a shape the kernels do not take (more than 128 tokens per chunk, S other
 than 128, head_dim other than 64 or 128) raises.
@@ -148,13 +149,11 @@ def layer_backward(mod, x: torch.Tensor, tr: dict, d_out: torch.Tensor, dt: torc
 
     Two streams.  This one: the o_proj products, the readout's backward, the chain's token
     statistics, the attention's backward, the chain's slot recursion and token gradients, the
-    key / value part of the head backward and the projections' products.  The side stream: the
-    chain's M_res recursion, a few long-lived workgroups that run beside the attention's backward
+    key / value part of the head backward, the small parameters' sums and the projections'
+    products.  The side stream: the chain's M_res recursion, a few long-lived workgroups that run beside the attention's backward
     (this stream holds the attention until they are resident, bolt3_wait_count), then the query
-    part of the head backward beside the chain's slot recursion and token gradients, and the
-    reductions to the small parameters.  Every buffer the side stream touches is allocated on this stream and held here
-    until this stream has waited for the side stream's last kernel; the side stream's own results
-    are marked as used on this stream."""
+    part of the head backward beside the chain's slot recursion and token gradients.  Every buffer the side stream touches is allocated on this stream and held here
+    until this stream has waited for the side stream's last kernel."""
     from .bolt3 import WAIT_POLLS, _n_cus, _started_counter   # (bolt3 imports this module)
     b, T, D = x.shape
     H, HKV, HD, S, C = mod.H, mod.HKV, mod.HD, mod.S, mod.C
@@ -241,24 +240,6 @@ def layer_backward(mod, x: torch.Tensor, tr: dict, d_out: torch.Tensor, dt: torc
     with torch.cuda.stream(aux):
         ha.parts = 1
         A.call("bolt3_heads_bwd", ha, dev)
-        small = {}
-        d_gam = o["d_gamma"].view(b, HKV, n_chunks).sum(dim=(0, 2))
-        if n_steps > 0:
-            d_gam = d_gam + cbuf["d_gamma"].view(n_steps, b, HKV, -1).sum(dim=(0, 1, 3))
-            # kappa: the slot bias is kappa * log(max(mass, 1)) (vsa_lm/config/bolt3.py:238-241)
-            dbias = o["d_bias"].sum(2).view(n_steps, b, HKV, G, S).sum(3)             # [step, b, HKV, S]
-            logm = tr["snap_mass"].clamp_min(1.0).log().view(n_steps, b, HKV, S)
-            small["kappa"] = (dbias * logm).sum(dim=(0, 1, 3))
-        else:
-            small["kappa"] = torch.zeros(HKV, device=dev)
-        # gamma = clamp(0.999 * sigmoid(log_gamma), 1e-3, 0.999); clamp passes its bounds inclusive
-        sg = torch.sigmoid(mod.log_gamma.detach().float().to(dev))
-        g0 = 0.999 * sg
-        inside = ((g0 >= 1e-3) & (g0 <= 0.999)).float()
-        small["log_gamma"] = d_gam * 0.999 * sg * (1.0 - sg) * inside
-        small["res_norm.weight"] = o["d_res_w"].sum(dim=(0, 1))
-        if has_norm:
-            small["q_norm.weight"] = d_qn.sum(0)
     if n_steps > 0:
         ca.kernels = A.CBWD_SLOT_REC
         A.call("bolt3_chain_bwd", ca, dev)
@@ -271,17 +252,35 @@ def layer_backward(mod, x: torch.Tensor, tr: dict, d_out: torch.Tensor, dt: torc
     widths = [H * HD, HKV * HD, HKV * HD, HKV, H]
     lins = (mod.q_proj, mod.k_proj, mod.v_proj, mod.beta_proj, mod.eta_proj)
     names = ("q_proj", "k_proj", "v_proj", "beta_proj", "eta_proj")
-    # the k norm's weight gradient and the biases' column sums of dz (accumulated in fp32, no fp32
-    # copy of dz) on the side stream, beside the projections' products
-    aux.wait_stream(main)
-    with torch.cuda.stream(aux):
-        if has_norm:
-            small["k_norm.weight"] = d_kn.sum(0)
-        off = 0
-        for name, lin, width in zip(names, lins, widths):
-            if lin.bias is not None:
-                small[f"{name}.bias"] = dz[:, off:off + width].sum(0, dtype=torch.float32)
-            off += width
+    # the small parameters' gradients (norm weights, kappa, gamma, the biases' column sums of dz), on
+    # this stream: beside the projections' products the launch takes 266 us instead of 49 (4 x 4096
+    # tokens, no faster as a whole) and short sequences pay for the hand-over (1.36 against 1.23 ms)
+    starts = [sum(widths[:i]) for i in range(len(widths))]
+    with_bias = [i for i, lin in enumerate(lins) if lin.bias is not None]
+    c0 = starts[with_bias[0]] if with_bias else 0
+    n_bias = starts[with_bias[-1]] + widths[with_bias[-1]] - c0 if with_bias else 0
+    sizes = dict(res_norm=HD, q_norm=HD, k_norm=HD, kappa=HKV, log_gamma=HKV, bias=n_bias)
+    buf = torch.empty(sum(sizes.values()), **f32)
+    sm = dict(zip(sizes, buf.split(list(sizes.values()))))
+    log_gamma = mod.log_gamma.detach().to(device=dev, dtype=torch.float32).contiguous()
+    pa = A.ParamGradsArgs()
+    pa.dtype, pa.B, pa.T, pa.H, pa.HKV, pa.HD, pa.S = A.dtype_code(dt), b, T, H, HKV, HD, S
+    pa.n_chunks, pa.n_qtiles, pa.n_steps, pa.n_blocks = n_chunks, (C + 31) // 32, n_steps, nb
+    pa.d_res_w, pa.d_gamma, pa.log_gamma = o["d_res_w"].data_ptr(), o["d_gamma"].data_ptr(), log_gamma.data_ptr()
+    if n_steps > 0:
+        pa.d_bias, pa.snap_mass, pa.d_gamma_chain = o["d_bias"].data_ptr(), tr["snap_mass"].data_ptr(), \
+            cbuf["d_gamma"].data_ptr()
+    if has_norm:
+        pa.d_qn_w, pa.d_kn_w = d_qn.data_ptr(), d_kn.data_ptr()
+    pa.dz, pa.dz_row_stride, pa.bias_col, pa.n_bias = dz.data_ptr(), dz.shape[1], c0, n_bias
+    pa.g_res_w, pa.g_qn_w, pa.g_kn_w, pa.g_bias, pa.g_kappa, pa.g_log_gamma = (
+        sm[k].data_ptr() for k in ("res_norm", "q_norm", "k_norm", "bias", "kappa", "log_gamma"))
+    A.call("bolt3_param_grads", pa, dev)
+    grads["kappa"], grads["log_gamma"], grads["res_norm.weight"] = sm["kappa"], sm["log_gamma"], sm["res_norm"]
+    if has_norm:
+        grads["q_norm.weight"], grads["k_norm.weight"] = sm["q_norm"], sm["k_norm"]
+    for i in with_bias:
+        grads[f"{names[i]}.bias"] = sm["bias"][starts[i] - c0:starts[i] - c0 + widths[i]]
     # one product each for dx and for the packed weight's gradient: rows q | k | v | beta | eta
     dx = F.linear(dz, side["wT"])
     dW = dz.t() @ x.reshape(b * T, D)
@@ -289,10 +288,6 @@ def layer_backward(mod, x: torch.Tensor, tr: dict, d_out: torch.Tensor, dt: torc
     for name, width in zip(names, widths):
         grads[f"{name}.weight"] = dW[off:off + width]
         off += width
-    main.wait_stream(aux)
-    for k, t in small.items():
-        t.record_stream(main)
-        grads[k] = t
     return dx.view(b, T, D), grads
 
 
