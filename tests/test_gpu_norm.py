@@ -46,6 +46,8 @@ def test_rms_norm_row_and_wave_kernels(rows, dim, offset, gpu):
     norm.weight.data = w
     with torch.no_grad():
         y, ref = norm(x), _torch_rms(x, w, 1e-6)
+        many = norm(x.repeat(1 + 300 // rows, 1))[:rows]      # enough rows for the other kernel
+    assert torch.equal(y, many)
     d = (y.float() - ref.float()).abs()
     assert bool((d <= ref.float().abs() * 2 ** -7 + 1e-30).all())
 

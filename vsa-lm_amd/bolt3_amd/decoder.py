@@ -765,7 +765,7 @@ class Bolt3Decoder:
     def _mlp(blk, x: torch.Tensor) -> torch.Tensor:
         """x + MLP(norm2(x)); the few rows of a one-token step stream the weights in two launches."""
         h = blk.norm2(x)
-        y = mlp_rows(blk.mlp, h, x)
+        y = mlp_rows(blk.mlp, h, x) if x.shape[1] == 1 else None
         return x + blk.mlp(h) if y is None else y
 
     # ------------------------------------------------------------ model-level API

@@ -39,16 +39,17 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(b3_rms_norm_args a) {
   }
 }
 
-// Few rows: one workgroup per row, the row in registers (NV pieces of 8 elements per thread), so that
-// the row is read once and by four wavefronts.  One row of 2560 in bf16, latency bound: 4.1 us a
-// launch in a captured decode step against 5.9 for the kernel above, where one wavefront reads
-// the row twice.
+// Few rows: one workgroup per row, the row read once into registers by four wavefronts (NV pieces
+// of 8 elements per thread).  The sum of squares keeps the order of the kernel above, so that both
+// give the same bits: the row passes through LDS and every wavefront adds all of it, lane l the
+// pieces l, l + 64, ...  One row of 2560 in bf16, latency bound: 4.1 us a launch in a captured
+// decode step against 5.9 for the kernel above, where one wavefront reads the row twice.
 constexpr int RN_NT = 256, RN_NV = 4;
 
 template <typename T, typename W>
 __global__ void __launch_bounds__(RN_NT) rms_norm_row_kernel(b3_rms_norm_args a) {
-  __shared__ float part[RN_NT / 64];
-  const int tid = threadIdx.x, n8 = a.dim / 8;
+  __shared__ __attribute__((aligned(16))) T row[8 * RN_NT * RN_NV];
+  const int tid = threadIdx.x, lane = tid & 63, n8 = a.dim / 8;
   const T* x = reinterpret_cast<const T*>(a.x) + (long long)blockIdx.x * a.x_row_stride;
   T* y = reinterpret_cast<T*>(a.y) + (long long)blockIdx.x * a.y_row_stride;
   Vec8<T> v[RN_NV];
@@ -59,21 +60,22 @@ __global__ void __launch_bounds__(RN_NT) rms_norm_row_kernel(b3_rms_norm_args a)
       v[q].load(x + 8 * (tid + RN_NT * q));
       w[q].load(reinterpret_cast<const W*>(a.w) + 8 * (tid + RN_NT * q));
     }
-  float ss = 0.f;
 #pragma unroll
   for (int q = 0; q < RN_NV; ++q)
-    if (tid + RN_NT * q < n8)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float f = v[q].get(e);
-        ss += f * f;
-      }
-  ss = wave_sum(ss);
-  if ((tid & 63) == 0) part[tid >> 6] = ss;
+    if (tid + RN_NT * q < n8) v[q].store(row + 8 * (tid + RN_NT * q));
   __syncthreads();
-  ss = 0.f;
+  float ss = 0.f;
+  for (int i = lane; i < n8; i += 64) {
+    Vec8<T> u;
+    u.load(row + 8 * i);
 #pragma unroll
-  for (int i = 0; i < RN_NT / 64; ++i) ss += part[i];
+    for (int e = 0; e < 8; ++e) {
+      const float f = u.get(e);
+      ss += f * f;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
   const float r = 1.0f / sqrtf(div_rn(ss, (float)a.dim) + a.eps);
 #pragma unroll
   for (int q = 0; q < RN_NV; ++q)
