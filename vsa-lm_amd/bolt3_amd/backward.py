@@ -157,7 +157,6 @@ def layer_backward(mod, x: torch.Tensor, tr: dict, d_out: torch.Tensor, dt: torc
     from .bolt3 import WAIT_POLLS, _n_cus, _started_counter   # (bolt3 imports this module)
     b, T, D = x.shape
     H, HKV, HD, S, C = mod.H, mod.HKV, mod.HD, mod.S, mod.C
-    G = H // HKV
     bh = b * HKV
     dev = x.device
     n_chunks = (T + C - 1) // C
