@@ -512,6 +512,18 @@ typedef struct {
 int bolt3_rows_linear(const b3_rows_linear_args* a, void* stream);
 
 /*
+ * out = round(round(silu(gate)) * up) over n bf16 elements (vsa_lm/surgery.py:210-211), n a multiple of
+ * 8, 16-byte aligned; out may be gate or up.
+ */
+typedef struct {
+  int64_t n;
+  const void* gate;
+  const void* up;
+  void* out;
+} b3_swiglu_args;
+int bolt3_swiglu(const b3_swiglu_args* a, void* stream);
+
+/*
  * RMSNorm of rows: y = (x * rsqrt(mean(x^2) + eps)) * w with an fp32 statistic, each product
  * rounded in fp32 and the result cast to the storage dtype (x's) once.  For the layers around
  * the Bolt-3 path in a hybrid stack (block norms, final norm, the softmax layers' q/k norms).

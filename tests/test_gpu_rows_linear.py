@@ -76,3 +76,20 @@ def test_mlp_rows_matches_module(M, gpu):
         many = torch.zeros(17, 1, 512, dtype=BF, device=gpu)
         assert mlp_rows(mlp, many, many) is None
     assert mlp_rows(mlp, h, res) is None             # gradients enabled
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 8), (3, 7, 1544), (2, 700, 1536)])
+def test_mlp_swiglu_equals_module(shape, gpu):
+    """One pass for silu(gate) * up, bit for bit the module's two (each of their roundings kept)."""
+    from bolt3_amd.layers import MLP, mlp_swiglu
+    g = torch.Generator(device=gpu).manual_seed(shape[1])
+    mlp = MLP(dict(dim=64, intermediate=shape[2])).to(gpu).to(BF)
+    h = (4 * torch.randn(*shape[:2], 64, generator=g, device=gpu)).to(BF)
+    h[0, 0, 0] = float("inf")
+    with torch.no_grad():
+        for p in mlp.parameters():
+            p.normal_(0.0, 0.5, generator=g)
+        got, ref = mlp_swiglu(mlp, h), mlp(h)
+        assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.nan_to_num(), ref.nan_to_num())
+        assert mlp_swiglu(mlp, h.float()) is None
+    assert mlp_swiglu(mlp, h) is None

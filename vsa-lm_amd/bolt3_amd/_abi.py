@@ -137,6 +137,10 @@ class RowsLinearArgs(C.Structure):
                 ("w2", p), ("bias", p), ("res", p), ("res_row_stride", i64), ("out", p), ("out_row_stride", i64)]
 
 
+class SwigluArgs(C.Structure):
+    _fields_ = [("n", i64), ("gate", p), ("up", p), ("out", p)]
+
+
 class RmsNormArgs(C.Structure):
     _fields_ = [("dtype", i32), ("rows", i64), ("dim", i32), ("x", p), ("x_row_stride", i64), ("w", p),
                 ("w_dtype", i32), ("y", p), ("y_row_stride", i64), ("eps", f32)]
@@ -185,7 +189,7 @@ EXPORTS = ("bolt3_attn_bwd", "bolt3_heads", "bolt3_heads_bwd", "bolt3_heads_bwd_
            "bolt3_decode",
            "bolt3_decode_layer", "bolt3_decode_layer_workspace_bytes", "bolt3_decode_workspace_bytes",
            "bolt3_param_grads",
-           "bolt3_rms_norm", "bolt3_rows_linear", "bolt3_slot_keys", "bolt3_step_advance", "bolt3_version", "bolt3_wait_count")
+           "bolt3_rms_norm", "bolt3_rows_linear", "bolt3_slot_keys", "bolt3_step_advance", "bolt3_swiglu", "bolt3_version", "bolt3_wait_count")
 
 _lib = None
 
@@ -204,7 +208,8 @@ def load():
                      ("bolt3_decode", DecodeArgs), ("bolt3_decode_layer", DecodeLayerArgs),
                      ("bolt3_slot_keys", SlotKeysArgs), ("bolt3_attn_bwd", AttnBwdArgs),
                      ("bolt3_rms_norm", RmsNormArgs), ("bolt3_rows_linear", RowsLinearArgs), ("bolt3_chain_bwd", ChainBwdArgs),
-                     ("bolt3_heads_bwd", HeadsBwdArgs), ("bolt3_param_grads", ParamGradsArgs)):
+                     ("bolt3_heads_bwd", HeadsBwdArgs), ("bolt3_param_grads", ParamGradsArgs),
+                     ("bolt3_swiglu", SwigluArgs)):
         fn = getattr(lib, name)
         fn.argtypes = [C.POINTER(st), p]
         fn.restype = C.c_int

@@ -29,7 +29,7 @@ import torch.nn.functional as F
 
 from . import _abi as A
 from .bolt3 import N_SINKS, Bolt3Attn, _check_dtype, _gout, _tout
-from .layers import mlp_rows
+from .layers import mlp_rows, mlp_swiglu
 
 DONE_CHECK_EVERY = 16      # tokens between the all-rows-done tests (the reference's period)
 
@@ -113,6 +113,13 @@ class AnchorCache:
 StaticKV = AnchorCache
 
 
+def _zeros(device, dtype, *shapes):
+    """Zero tensors of the given shapes, cleared in one launch."""
+    out = [torch.empty(s, dtype=dtype, device=device) for s in shapes]
+    torch._foreach_zero_(out)
+    return out
+
+
 class Bolt3LayerState(MutableMapping):
     """Decoder state of one Bolt-3 layer in preallocated device buffers.
 
@@ -138,18 +145,16 @@ class Bolt3LayerState(MutableMapping):
         self.B, self.C, self.S, self.HKV, self.HD, self.dtype = B, C, S, HKV, HD, dtype
         self._ly = ly
         self.cap = 4 * C
-        self.win_kr = torch.zeros(B, HKV, self.cap, HD, dtype=dtype, device=device)
-        self.win_kp = torch.zeros_like(self.win_kr)
-        self.win_v = torch.zeros_like(self.win_kr)
-        self.win_b = torch.zeros(B, HKV, self.cap, device=device)
-        self.win_pos = torch.zeros(self.cap, device=device)
-        self.sink_k = torch.zeros(B, HKV, N_SINKS, HD, dtype=dtype, device=device)
-        self.sink_v = torch.zeros_like(self.sink_k)
-        self.n_sink = 0
         bh = B * HKV
-        self.slots = ly._empty_slots(bh, dtype, device)
-        self.slot_k = torch.zeros(bh, S, HD, dtype=dtype, device=device)
-        self.slot_bias = torch.zeros(bh, S, device=device)
+        win, sink, slot = (B, HKV, self.cap, HD), (B, HKV, N_SINKS, HD), (bh, S, HD)
+        # one zero fill per dtype instead of one per tensor (some 4 us each, in every layer of a prefill)
+        self.win_kr, self.win_kp, self.win_v, self.sink_k, self.sink_v, ak, av, self.slot_k = _zeros(
+            device, dtype, win, win, win, sink, sink, slot, slot, slot)
+        self.win_b, self.win_pos, util, pm, self.slot_bias = _zeros(
+            device, torch.float32, (B, HKV, self.cap), (self.cap,), (bh, S), (bh, S), (bh, S))
+        self.n_sink = 0
+        self.slots = dict(ak=ak, av=av, mass=torch.ones(bh, S, dtype=torch.float32, device=device), util=util, pm=pm,
+                          act=torch.zeros(bh, S, dtype=torch.uint8, device=device))
         self.has_slots = False
         self.n_filled = 0
         self.prev = (0, 0)          # (start, length) in the ring
@@ -239,7 +244,8 @@ class Bolt3LayerState(MutableMapping):
         bh = B * HKV
 
         def put(dst, src, shape):
-            dst.copy_(src.detach().reshape(shape).to(device=dev, dtype=dst.dtype))
+            src = src.detach()
+            dst.copy_(src if src.shape == torch.Size(shape) else src.reshape(shape))
 
         if d.get("ak") is None:
             for k, v in self._ly._empty_slots(bh, dt, dev).items():
@@ -766,7 +772,10 @@ class Bolt3Decoder:
         """x + MLP(norm2(x)); the few rows of a one-token step stream the weights in two launches."""
         h = blk.norm2(x)
         y = mlp_rows(blk.mlp, h, x) if x.shape[1] == 1 else None
-        return x + blk.mlp(h) if y is None else y
+        if y is not None:
+            return y
+        y = mlp_swiglu(blk.mlp, h)
+        return x + (blk.mlp(h) if y is None else y)
 
     # ------------------------------------------------------------ model-level API
 
@@ -825,7 +834,7 @@ class Bolt3Decoder:
                     x = x + self._bolt3_prefill(blk.vsa, h, states[li], kv[li], rec)
                 else:
                     x = x + self._anchor_layer(blk.attn, h, 0, kv[li])
-                x = x + blk.mlp(blk.norm2(x))
+                x = self._mlp(blk, x)
             s_last = ((t - 1) // self.C) * self.C
             return m.norm(x[:, s_last:]), states, kv
 

@@ -7,7 +7,7 @@ path (the softmax-anchor layers and the model container that
 ``Bolt3Decoder`` walks); they run as PyTorch ops on the device, except
 ``RMSNorm``, whose device forward is the library's ``bolt3_rms_norm`` (one pass
 per row instead of the torch ops' six; CPU tensors keep the torch ops), and the
-MLP of a one-token decode step (``mlp_rows``).
+decoder's MLPs (``mlp_rows`` for a one-token step, ``mlp_swiglu``).
   RMSNorm      -- vsa_lm/surgery.py:43-53
   rope_inv_freq-- vsa_lm/surgery.py:56-72
   RoPE         -- vsa_lm/surgery.py:80-93
@@ -151,6 +151,26 @@ def mlp_rows(mlp: nn.Module, h: torch.Tensor, res: torch.Tensor) -> torch.Tensor
     a.res, a.res_row_stride, a.out, a.out_row_stride = r.data_ptr(), r.stride(0), out.data_ptr(), D
     A.call("bolt3_rows_linear", a, h.device)
     return out.view(h.shape)
+
+
+def mlp_swiglu(mlp: nn.Module, h: torch.Tensor) -> torch.Tensor | None:
+    """mlp(h) with SwiGLU as one pass over the two projections' outputs instead of the module's two (the
+    same roundings); None where it does not apply (gradients, autocast, another MLP, not bf16)."""
+    if (type(mlp) is not MLP or not h.is_cuda or h.dtype != torch.bfloat16 or type(h) is not torch.Tensor or
+            torch.is_grad_enabled() or torch.is_autocast_enabled(h.device.type) or mlp._forward_hooks or
+            mlp._forward_pre_hooks):
+        return None
+    g, u = mlp.gate_proj(h), mlp.up_proj(h)
+    if (g.dtype != torch.bfloat16 or u.dtype != g.dtype or u.shape != g.shape or u.device != g.device or
+            not g.is_contiguous() or not u.is_contiguous() or g.numel() % 8 or g.data_ptr() % 16 or u.data_ptr() % 16 or
+            type(g) is not torch.Tensor or type(u) is not torch.Tensor):
+        return mlp.down_proj(F.silu(g) * u)
+    from . import _abi as A
+    act = torch.empty_like(g)
+    a = A.SwigluArgs()
+    a.n, a.gate, a.up, a.out = g.numel(), g.data_ptr(), u.data_ptr(), act.data_ptr()
+    A.call("bolt3_swiglu", a, h.device)
+    return mlp.down_proj(act)
 
 
 class SoftmaxAttn(nn.Module):
