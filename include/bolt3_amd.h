@@ -524,6 +524,24 @@ typedef struct {
 int bolt3_swiglu(const b3_swiglu_args* a, void* stream);
 
 /*
+ * n copies of rows of contiguous bytes in one launch.  Each piece: rows >= 0 rows of row_bytes >= 0
+ * bytes, src_stride and dst_stride bytes apart; no dst may overlap another piece's dst or any src.
+ * B3_ERR_UNSUPPORTED where a piece has 2^31 units or more (16 bytes where addresses, strides and
+ * row_bytes are multiples of 16, else 4 or 1).
+ */
+#define B3_COPY_MAX 24
+typedef struct {
+  int64_t rows, row_bytes, src_stride, dst_stride;
+  const void* src;
+  void* dst;
+} b3_copy_piece;
+typedef struct {
+  int32_t n;
+  b3_copy_piece piece[B3_COPY_MAX];
+} b3_copy_pieces_args;
+int bolt3_copy_pieces(const b3_copy_pieces_args* a, void* stream);
+
+/*
  * RMSNorm of rows: y = (x * rsqrt(mean(x^2) + eps)) * w with an fp32 statistic, each product
  * rounded in fp32 and the result cast to the storage dtype (x's) once.  For the layers around
  * the Bolt-3 path in a hybrid stack (block norms, final norm, the softmax layers' q/k norms).

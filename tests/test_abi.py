@@ -106,7 +106,8 @@ STRUCTS = {"b3_heads_args": A.HeadsArgs, "b3_chain_args": A.ChainArgs, "b3_attn_
            "b3_slot_keys_args": A.SlotKeysArgs, "b3_attn_bwd_args": A.AttnBwdArgs,
            "b3_rms_norm_args": A.RmsNormArgs, "b3_chain_bwd_args": A.ChainBwdArgs,
            "b3_heads_bwd_args": A.HeadsBwdArgs, "b3_rows_linear_args": A.RowsLinearArgs,
-           "b3_param_grads_args": A.ParamGradsArgs, "b3_swiglu_args": A.SwigluArgs}
+           "b3_param_grads_args": A.ParamGradsArgs, "b3_swiglu_args": A.SwigluArgs,
+           "b3_copy_piece": A.CopyPiece, "b3_copy_pieces_args": A.CopyPiecesArgs}
 
 
 def _flat_fields(st, prefix=""):

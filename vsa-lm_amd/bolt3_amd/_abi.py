@@ -141,6 +141,17 @@ class SwigluArgs(C.Structure):
     _fields_ = [("n", i64), ("gate", p), ("up", p), ("out", p)]
 
 
+COPY_MAX = 24             # B3_COPY_MAX
+
+
+class CopyPiece(C.Structure):
+    _fields_ = [("rows", i64), ("row_bytes", i64), ("src_stride", i64), ("dst_stride", i64), ("src", p), ("dst", p)]
+
+
+class CopyPiecesArgs(C.Structure):
+    _fields_ = [("n", i32), ("piece", CopyPiece * COPY_MAX)]
+
+
 class RmsNormArgs(C.Structure):
     _fields_ = [("dtype", i32), ("rows", i64), ("dim", i32), ("x", p), ("x_row_stride", i64), ("w", p),
                 ("w_dtype", i32), ("y", p), ("y_row_stride", i64), ("eps", f32)]
@@ -186,10 +197,11 @@ class ParamGradsArgs(C.Structure):
 EXPORTS = ("bolt3_attn_bwd", "bolt3_heads", "bolt3_heads_bwd", "bolt3_heads_bwd_blocks", "bolt3_chain",
            "bolt3_chain_bwd", "bolt3_chain_bwd_workspace_bytes",
            "bolt3_chain_noalloc", "bolt3_chain_workspace_bytes", "bolt3_chunk_attn",
-           "bolt3_decode",
+           "bolt3_copy_pieces", "bolt3_decode",
            "bolt3_decode_layer", "bolt3_decode_layer_workspace_bytes", "bolt3_decode_workspace_bytes",
            "bolt3_param_grads",
-           "bolt3_rms_norm", "bolt3_rows_linear", "bolt3_slot_keys", "bolt3_step_advance", "bolt3_swiglu", "bolt3_version", "bolt3_wait_count")
+           "bolt3_rms_norm", "bolt3_rows_linear", "bolt3_slot_keys", "bolt3_step_advance",
+           "bolt3_swiglu", "bolt3_version", "bolt3_wait_count")
 
 _lib = None
 
@@ -209,7 +221,8 @@ def load():
                      ("bolt3_slot_keys", SlotKeysArgs), ("bolt3_attn_bwd", AttnBwdArgs),
                      ("bolt3_rms_norm", RmsNormArgs), ("bolt3_rows_linear", RowsLinearArgs), ("bolt3_chain_bwd", ChainBwdArgs),
                      ("bolt3_heads_bwd", HeadsBwdArgs), ("bolt3_param_grads", ParamGradsArgs),
-                     ("bolt3_swiglu", SwigluArgs)):
+                     ("bolt3_swiglu", SwigluArgs),
+                     ("bolt3_copy_pieces", CopyPiecesArgs)):
         fn = getattr(lib, name)
         fn.argtypes = [C.POINTER(st), p]
         fn.restype = C.c_int

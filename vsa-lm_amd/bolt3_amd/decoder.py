@@ -120,6 +120,64 @@ def _zeros(device, dtype, *shapes):
     return out
 
 
+def _row_form(shape, strides):
+    """(elements of a contiguous row, elements between rows) of a strided tensor whose elements are
+    rows of one length at one distance; None if they are not.  One row: distance = its length."""
+    dims = [(n, st) for n, st in zip(shape, strides) if n != 1]
+    row = 1
+    while dims and dims[-1][1] == row:
+        row *= dims.pop()[0]
+    if not dims:
+        return row, row
+    step = dims[-1][1]
+    at = step
+    for n, st in reversed(dims):
+        if st != at:
+            return None
+        at = n * st
+    return row, step
+
+
+def _copy_piece(dst: torch.Tensor, src: torch.Tensor):
+    """(rows, row bytes, src and dst bytes between rows) of dst.copy_(src) as a plain copy of bytes, or
+    None: the tensors have one shape and either the same row length or one of them is a single row."""
+    if (src.device != dst.device or src.dtype != dst.dtype or src.shape != dst.shape or type(src) is not torch.Tensor or
+            src.numel() == 0 or src.numel() >= 1 << 30 or src.is_neg()):
+        return None
+    a, b = _row_form(src.shape, src.stride()), _row_form(dst.shape, dst.stride())
+    if a is None or b is None:
+        return None
+    n, row = src.numel(), min(a[0], b[0])
+    if any(r != row and r != n for r, _ in (a, b)):
+        return None
+    e = dst.element_size()
+    return n // row, row * e, (a[1] if a[0] == row else row) * e, (b[1] if b[0] == row else row) * e
+
+
+def _copy_all(pairs):
+    """dst.copy_(src) for every pair, those that are plain copies on one GPU in one launch (a prefill's
+    layer has 17, some 4.4 us each); one after another where a source shares memory with a target."""
+    own = {dst.untyped_storage().data_ptr() for dst, _ in pairs}
+    fused = [] if any(src.untyped_storage().data_ptr() in own for _, src in pairs) else pairs
+    pieces = []
+    for dst, src in fused:
+        f = _copy_piece(dst, src) if dst.is_cuda else None
+        if f is not None and len(pieces) < A.COPY_MAX:
+            pieces.append((dst, src, f))
+    done = {id(dst) for dst, _, _ in pieces}
+    for dst, src in pairs:
+        if id(dst) not in done:
+            dst.copy_(src)
+    if pieces:
+        a = A.CopyPiecesArgs()
+        a.n = len(pieces)
+        for i, (dst, src, f) in enumerate(pieces):
+            q = a.piece[i]
+            q.rows, q.row_bytes, q.src_stride, q.dst_stride = f
+            q.src, q.dst = src.data_ptr(), dst.data_ptr()
+        A.call("bolt3_copy_pieces", a, pieces[0][0].device)
+
+
 class Bolt3LayerState(MutableMapping):
     """Decoder state of one Bolt-3 layer in preallocated device buffers.
 
@@ -243,9 +301,11 @@ class Bolt3LayerState(MutableMapping):
         dev = self.win_kr.device
         bh = B * HKV
 
+        pairs = []
+
         def put(dst, src, shape):
             src = src.detach()
-            dst.copy_(src if src.shape == torch.Size(shape) else src.reshape(shape))
+            pairs.append((dst, src if src.shape == torch.Size(shape) else src.reshape(shape)))
 
         if d.get("ak") is None:
             for k, v in self._ly._empty_slots(bh, dt, dev).items():
@@ -258,7 +318,6 @@ class Bolt3LayerState(MutableMapping):
                 put(self.slots[k], d[k], (bh, S))
             put(self.slots["act"], d["act"].to(torch.uint8), (bh, S))
             self.has_slots = True
-            self._refresh_slot_keys()
         self.n_filled = int(d.get("n_filled") or 0)
         if d.get("sink_k") is None:
             self.n_sink = 0
@@ -284,6 +343,9 @@ class Bolt3LayerState(MutableMapping):
                 self.prev = (start, n)
             else:
                 self.cur = (start, n)
+        _copy_all(pairs)
+        if self.has_slots:
+            self._refresh_slot_keys()
 
     def _refresh_slot_keys(self):
         ly = self._ly
