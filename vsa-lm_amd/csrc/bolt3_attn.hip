@@ -291,11 +291,39 @@ __global__ void __launch_bounds__(512) attn_kernel(b3_attn_args a, int QW) {
           for (int i = 0; i < 8; ++i) sV[(c8 + i) * sm.VS + r] = vv[i];
         }
       } else {
-        for (int it = tid; it < KB * HD; it += nthreads) {
-          const int r = it / HD, c = it % HD;
-          const bool ok = k0 + r < sg.len;
-          sK[r * sm.KS + c] = ok ? kbase[(long long)(k0 + r) * HD + c] : 0.f;
-          sV[c * sm.VS + r] = ok ? vbase[(long long)(k0 + r) * HD + c] : 0.f;
+        // 16-byte loads, three units of a thread in flight (a workgroup of 192 threads then waits for
+        // memory once per block at HD = 64), where the rows are aligned
+        constexpr int UN = 3, V4 = HD / 4;
+        if ((reinterpret_cast<uintptr_t>(kbase) | reinterpret_cast<uintptr_t>(vbase)) % 16 == 0) {
+          for (int it0 = tid; it0 < KB * V4; it0 += UN * nthreads) {
+            f32x4 kv[UN], vv[UN];
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+              const int it = it0 + u * nthreads, r = it / V4, c = 4 * (it % V4);
+              kv[u] = vv[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+              if (it < KB * V4 && k0 + r < sg.len) {
+                kv[u] = *reinterpret_cast<const f32x4*>(kbase + (long long)(k0 + r) * HD + c);
+                vv[u] = *reinterpret_cast<const f32x4*>(vbase + (long long)(k0 + r) * HD + c);
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+              const int it = it0 + u * nthreads, r = it / V4, c = 4 * (it % V4);
+              if (it < KB * V4)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  sK[r * sm.KS + c + e] = kv[u][e];
+                  sV[(c + e) * sm.VS + r] = vv[u][e];
+                }
+            }
+          }
+        } else {
+          for (int it = tid; it < KB * HD; it += nthreads) {
+            const int r = it / HD, c = it % HD;
+            const bool ok = k0 + r < sg.len;
+            sK[r * sm.KS + c] = ok ? kbase[(long long)(k0 + r) * HD + c] : 0.f;
+            sV[c * sm.VS + r] = ok ? vbase[(long long)(k0 + r) * HD + c] : 0.f;
+          }
         }
       }
       if (tid < KB) sm.bias[tid] = (sg.kind == 1 && k0 + tid < sg.len) ? slot_b[k0 + tid] : 0.f;
@@ -312,7 +340,7 @@ __global__ void __launch_bounds__(512) attn_kernel(b3_attn_args a, int QW) {
           mma_bf16(s, av, qf.v[ks]);
         }
       } else {
-#pragma unroll 8
+#pragma unroll F32_UNROLL<HD>
         for (int ks = 0; ks < HD / 2; ++ks) mma_f32(s, sK[n * sm.KS + 2 * ks + h], qf.v[ks]);
       }
       float bm = -INFINITY;
@@ -431,7 +459,7 @@ __global__ void __launch_bounds__(512) attn_kernel(b3_attn_args a, int QW) {
           mma_bf16(rr[db], al, rf.v[ks]);
         }
       } else {
-#pragma unroll 8
+#pragma unroll F32_UNROLL<HD>
         for (int ks = 0; ks < HD / 2; ++ks) mma_f32(rr[db], sm.mf()[(2 * ks + h) * sm.MF + d], rf.v[ks]);
       }
     }
@@ -1421,6 +1449,14 @@ static int launch_attn(const b3_attn_args& a, hipStream_t st) {
         (nw == 2 || nw == 4 || nw == 8)) {
       if (a.score_round) launch_fwd2<HD, true, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
       else launch_fwd2<HD, false, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
+      return (int)hipGetLastError();
+    }
+  }
+  if constexpr (!St<T>::is_bf16) {
+    // fp32: one query tile per head and workgroup where two would leave CUs without one (a wavefront's
+    // own work is the same, and so are the bits).  1 x 1024 tokens, 3 kv heads of 3: 96 workgroups for 48.
+    if (QW == 2 && G >= 2 && (long long)grid.x * grid.y * grid.z < 256) {
+      hipLaunchKernelGGL((attn_kernel<T, HD>), dim3((qlen + 31) / 32, grid.y, grid.z), dim3(64 * G), 0, st, a, 1);
       return (int)hipGetLastError();
     }
   }

@@ -194,7 +194,7 @@ template <int HD>
 __device__ __forceinline__ void mm_rows_frag(f32x16& acc, const float* rows, int rs, int row0,
                                              const Frag<float, HD>& f, int lane) {
   const int m = row0 + (lane & 31), h = lane >> 5;
-#pragma unroll 8
+#pragma unroll F32_UNROLL<HD>
   for (int ks = 0; ks < HD / 2; ++ks) mma_f32(acc, rows[m * rs + 2 * ks + h], f.v[ks]);
 }
 
@@ -1985,7 +1985,7 @@ __global__ void __launch_bounds__(MT) gersh_kernel(b3_chain_args a) {
         Frag<T, HD> fi;
         fi.load(kr, 32 * ti + n, l, lane);
         // rows i of tile ti as the A operand: same fragment layout as a B fragment
-#pragma unroll 8
+#pragma unroll F32_UNROLL<HD>
         for (int ks = 0; ks < HD / 2; ++ks) mma_f32(acc, fi.v[ks], fj.v[ks]);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -2142,7 +2142,7 @@ __global__ void __launch_bounds__(MT) mres_kernel(b3_chain_args a) {
               mma_bf16(acc, lo, in.fj.v[ks]);
             }
           } else {
-#pragma unroll 8
+#pragma unroll F32_UNROLL<HD>
             for (int ks = 0; ks < HD / 2; ++ks) mma_f32(acc, sm.mt[n * Sm::MS + 2 * ks + h], in.fj.v[ks]);
           }
 #pragma unroll
@@ -2217,7 +2217,7 @@ __global__ void __launch_bounds__(MT) mres_kernel(b3_chain_args a) {
               mma_bf16(acc, lo, fj.v[ks]);
             }
           } else {
-#pragma unroll 8
+#pragma unroll F32_UNROLL<HD>
             for (int ks = 0; ks < HD / 2; ++ks) mma_f32(acc, sm.mt[n * Sm::MS + 2 * ks + h], fj.v[ks]);
           }
           const float inj = j < l ? inv_all[row + j] : 0.f;

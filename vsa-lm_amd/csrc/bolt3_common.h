@@ -304,4 +304,10 @@ static inline int cu_count() {
   return n;
 }
 
+// Steps of an fp32 product's loop over HD / 2 that are unrolled.  A fragment indexed by a running count
+// lies in scratch memory; whole at HD = 64 it stays in registers, which two fragments of HD = 128 do not
+// fit.  1 x 1024 tokens, SmolLM shape, whole against 8: decide_kernel 405 -> 336 us, attn_kernel (with
+// its wider loads and narrower workgroups) 145 -> 76, gersh_kernel 37 -> 26, mres_kernel 48 -> 45.
+template <int HD> constexpr int F32_UNROLL = HD == 64 ? 32 : 8;
+
 }  // namespace b3
