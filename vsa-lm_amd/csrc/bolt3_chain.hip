@@ -1421,45 +1421,37 @@ __global__ void __launch_bounds__(DT) decide_kernel(b3_chain_args a) {
     // steady steps read the slots
     bool has = false;
     if (__builtin_expect(nf == 0, 0)) {
-      // score = unbiased variance of normalize(v); four threads per token, each with a quarter of
-      // its features in registers (one thread per token, reading the row three times, left 6 of
-      // the 8 wavefronts idle: the step took 31 us at HD = 128, now 21; bound by the ordered sums)
-      constexpr int NQ = HD / 4;
-      for (int j = tid >> 2; j < ((l + 127) & ~127); j += DT / 4) {
-        float x[NQ];
+      // score = unbiased variance of normalize(v), one thread per token: the scores order the slots and
+      // every later tie follows that order, so their bits matter (four threads per token with the sums
+      // handed on in order took 21 us instead of 31, but differed by an ulp in 9 of 2000 tokens)
+      const int j = tid;
+      if (j < l) {
+        const T* vr = v + (long long)j * HD;
+        float ss = 0.f;
+        for (int d = 0; d < HD; d += 8) {
+          float x[8];
+          ld8(vr + d, x);
 #pragma unroll
-        for (int d = 0; d < NQ; d += 8) {
-          if (j < l) ld8(v + (long long)j * HD + (tid & 3) * NQ + d, x + d);
-          else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[d + i] = 0.f;
-          }
+          for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
         }
-        // every sum runs through the row's features in order, from one thread of the four to the
-        // next (the scores order the slots, and the order among equal keep values follows them)
-        auto chain = [&](auto&& add) {
-          float s = 0.f;
+        const float nrm = fmaxf(sqrtf(ss), 1e-12f);
+        float mean = 0.f;
+        for (int d = 0; d < HD; d += 8) {
+          float x[8];
+          ld8(vr + d, x);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            float t = q == 0 ? 0.f : __shfl(s, (lane & ~3) + q - 1, 64);
-#pragma unroll
-            for (int i = 0; i < NQ; ++i) add(t, x[i]);
-            s = t;
-          }
-          return __shfl(s, lane | 3, 64);
-        };
-        const float nrm = fmaxf(sqrtf(chain([](float& t, float u) { t += u * u; })), 1e-12f);
-#pragma unroll
-        for (int i = 0; i < NQ; ++i) x[i] = div_rn(x[i], nrm);
-        const float mean = chain([](float& t, float u) { t += u; }) / (float)HD;
-        const float var = chain([&](float& t, float u) {
-          const float c = u - mean;
-          t += c * c;
-        });
-        if (j < l && (tid & 3) == 0) {
-          sm.score[j] = var / (float)(HD - 1);
-          sm.rel[j] = 0.15f;
+          for (int i = 0; i < 8; ++i) mean += div_rn(x[i], nrm);
         }
+        mean /= (float)HD;
+        float var = 0.f;
+        for (int d = 0; d < HD; d += 8) {
+          float x[8];
+          ld8(vr + d, x);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) { const float u = div_rn(x[i], nrm) - mean; var += u * u; }
+        }
+        sm.score[j] = var / (float)(HD - 1);
+        sm.rel[j] = 0.15f;
       }
     } else {
       if constexpr (BF) has = score_phase16<HD>(sm, td, td_ready, kr, kp, v, l, steady, scale, wave, lane, log);

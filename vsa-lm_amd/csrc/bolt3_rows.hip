@@ -25,9 +25,9 @@ extern "C" int bolt3_rows_linear(const b3_rows_linear_args* a, void* stream) {
 }
 
 namespace b3 {
-// out = round(round(silu(gate)) * up), elementwise: the SwiGLU between the
-// library's products of a prompt or a large batch.  Bound by its three passes over memory: 37 us
-// for 4000 x 9728 (233 MB) against 68 us for torch's two kernels, which write and read silu(gate) between.
+// out = round(round(silu(gate)) * up), elementwise: the SwiGLU between the library's products of a
+// prompt or a large batch.  Bound by its three passes over memory: 37 us for 4000 x 9728 (233 MB)
+// against 68 us for torch's two kernels, which write and read silu(gate) between.
 __global__ void __launch_bounds__(256) swiglu_kernel(const uint16_t* g, const uint16_t* u, uint16_t* out, long long n8) {
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
     const u16x8 a = *reinterpret_cast<const u16x8*>(g + 8 * i), b = *reinterpret_cast<const u16x8*>(u + 8 * i);
