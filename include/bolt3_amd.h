@@ -430,8 +430,9 @@ int64_t bolt3_decode_workspace_bytes(int32_t B, int32_t H, int32_t HKV, int32_t 
  * A whole one-token decode layer step in bf16: the packed input projection
  * x . W_in^T + b_in (W_in rows q | k | v | beta | eta, zero rows padding to n_in), the
  * bolt3_decode step on that row, then out = y . W_out^T + b_out (rounded, then + res where res
- * is set).  The projections stream each weight once; the projected rows (B <= 16) or the fp32
- * partial products of 512-column chunks (B > 16) go through proj_work.
+ * is set).  The projections stream each weight once and add 512-column chunks of K in order, so
+ * that a row's bits do not depend on B; the projected rows (few) or the chunks' fp32 partial
+ * products (more) go through proj_work.
  * Replaces vsa_lm/config/bolt3.py:346-402 for t_s == 1 together with the q/k/v/beta/eta
  * projections it calls (:59-66, :349) and o_proj (:400-402).
  */

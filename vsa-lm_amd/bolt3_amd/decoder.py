@@ -466,6 +466,10 @@ class Bolt3Decoder:
         # bf16 one-token steps run as one bolt3_decode_layer call (projections included); False
         # keeps the projections in torch around bolt3_decode (the tests compare the two)
         self.fuse_projections = True
+        # True: the MLP of a one-token step of up to 16 rows in two launches that stream the weights
+        # (layers.mlp_rows) instead of the module's products; the sums then run in another order than
+        # in every other step, and the slot decisions that follow are those of other roundings
+        self.fuse_mlp = False
         # generate_batch replays a captured graph of the one-token step when the stack allows it
         self.use_graphs = True
         self._anchor_packs: dict = {}
@@ -829,11 +833,10 @@ class Bolt3Decoder:
         out = ly.o_proj(y.transpose(1, 2).reshape(b, t, ly.H * ly.HD))
         return out if res is None else res + out
 
-    @staticmethod
-    def _mlp(blk, x: torch.Tensor) -> torch.Tensor:
-        """x + MLP(norm2(x)); the few rows of a one-token step stream the weights in two launches."""
+    def _mlp(self, blk, x: torch.Tensor) -> torch.Tensor:
+        """x + MLP(norm2(x)), by default with the module's own products whatever the number of rows."""
         h = blk.norm2(x)
-        y = mlp_rows(blk.mlp, h, x) if x.shape[1] == 1 else None
+        y = mlp_rows(blk.mlp, h, x) if self.fuse_mlp and x.shape[1] == 1 else None
         if y is not None:
             return y
         y = mlp_swiglu(blk.mlp, h)

@@ -7,7 +7,7 @@ path (the softmax-anchor layers and the model container that
 ``Bolt3Decoder`` walks); they run as PyTorch ops on the device, except
 ``RMSNorm``, whose device forward is the library's ``bolt3_rms_norm`` (one pass
 per row instead of the torch ops' six; CPU tensors keep the torch ops), and the
-decoder's MLPs (``mlp_rows`` for a one-token step, ``mlp_swiglu``).
+decoder's MLPs (``mlp_swiglu``; ``mlp_rows`` for a one-token step on request).
   RMSNorm      -- vsa_lm/surgery.py:43-53
   rope_inv_freq-- vsa_lm/surgery.py:56-72
   RoPE         -- vsa_lm/surgery.py:80-93

@@ -13,8 +13,8 @@
 //   fp32: decode_split_kernel, grid (ceil(keys / 128) + HD/32, B*HKV), 128-key pieces and
 //     32-row readout pieces in parallel with fp32 MFMAs, then decode_combine_kernel, grid
 //     (B*HKV), merges the partial softmaxes and finishes the readout.
-// bolt3_decode_layer (bf16) adds the two projections around these: up to 16 rows in one kernel
-// each (bolt3_rows.h); above, rowproj_kernel streams a weight once per step and leaves fp32
+// bolt3_decode_layer (bf16) adds the two projections around these: up to ROWS_PROJ rows in one
+// kernel each (bolt3_rows.h); above, with the same bits, rowproj_kernel streams a weight once per step and leaves fp32
 // partial products per K chunk; the prep kernel sums those of the input projection and
 // proj_reduce_kernel those of o_proj.
 #include <algorithm>
@@ -1191,7 +1191,7 @@ extern "C" int bolt3_decode(const b3_decode_args* a, void* stream) {
 extern "C" int64_t bolt3_decode_layer_workspace_bytes(int32_t B, int32_t d_model, int32_t n_in, int32_t hd_total,
                                                       int32_t n_out) {
   if (B <= 0 || d_model <= 0 || n_in <= 0 || hd_total <= 0 || n_out <= 0) return 0;
-  if (B <= b3::ROWS_MAX) return ((int64_t)B * n_in * 2 + 15) / 16 * 16;   // the projected rows, rounded
+  if (B <= b3::ROWS_PROJ) return ((int64_t)B * n_in * 2 + 15) / 16 * 16;   // the projected rows, rounded
   const long long a = b3::proj_parts_floats(B, n_in, d_model), b = b3::proj_parts_floats(B, n_out, hd_total);
   return (int64_t)(a > b ? a : b) * 4;
 }
@@ -1218,7 +1218,7 @@ extern "C" int bolt3_decode_layer(const b3_decode_layer_args* a, void* stream) {
     return B3_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   using u16 = const uint16_t*;
-  if (d.B <= b3::ROWS_MAX) {
+  if (d.B <= b3::ROWS_PROJ) {
     b3_decode_args step = d;
     step.lin = a->proj_work;
     const b3::RowsArgs pin{static_cast<u16>(a->x), a->x_row_stride, static_cast<u16>(a->w_in), nullptr,
