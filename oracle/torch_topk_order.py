@@ -271,7 +271,8 @@ def topk_order_wave(values, k: int, largest: bool = True) -> tuple[list[int], bo
 
 
 def topk_order_levels(values, k: int, largest: bool = True) -> tuple[list[int], bool]:
-    """The kernel's restatement, level by level.  Returns (indices, depth_limit_reached)."""
+    """The kernel's restatement, level by level.  Returns (indices, depth_limit_reached); when the
+    flag is set the indices are still those of the k first values, sorted by value."""
     n = len(values)
     if k <= 0:
         return [], False
@@ -280,10 +281,12 @@ def topk_order_levels(values, k: int, largest: bool = True) -> tuple[list[int], 
     full = [order_key(v, largest) for v in values]
     key = np.array([sum(o < c for o in full) for c in full], dtype=np.int64)     # dense keys
     idx = np.arange(n)
+    limit = False
     f, l, depth = 0, n, 2 * _lg(n)
     while l - f > SELECT_THRESHOLD:
         if depth == 0:
-            return [int(i) for i in idx[:k]], True
+            limit = True
+            break
         depth -= 1
         cut = _partition_wave(key, idx, f, l)
         f, l = (cut, l) if cut <= k - 1 else (f, cut)
@@ -292,7 +295,8 @@ def topk_order_levels(values, k: int, largest: bool = True) -> tuple[list[int], 
     ranges, depth = [(0, ks)], 2 * _lg(ks) if ks > 1 else 0
     while any(b - a > SORT_THRESHOLD for a, b in ranges):
         if depth == 0:
-            return [int(i) for i in idx[:k]], True
+            limit = True
+            break
         depth -= 1
         level = []
         for a, b in ranges:            # disjoint: the kernel partitions them in one pass
@@ -305,7 +309,7 @@ def topk_order_levels(values, k: int, largest: bool = True) -> tuple[list[int], 
     out = [int(idx[k - 1])] * k
     for p in range(ks):
         out[int(key[p]) + int((key[:p] == key[p]).sum())] = int(idx[p])
-    return out, False
+    return out, limit
 
 
 def tie_in_prefix(sorted_values, n: int) -> bool:

@@ -305,7 +305,7 @@ __device__ __forceinline__ int count_below(const double* keys, int i0, int i1, d
 // the same utility, orders its 128 slots this way; the chain of levels bounds it: 14 us (HD = 128)
 // where one range after the other, with its elements in LDS as 64-bit keys, took 41 us.
 // A depth limit reached (heap fallback of the library, not restated) sets bit 0 of the returned
-// flags.
+// flags: the k elements are then those that come first, ordered as the ranks left them.
 __device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 __device__ __forceinline__ uint32_t pk_key(uint32_t e) { return e >> 8; }
@@ -510,7 +510,8 @@ __device__ int tie_order_wave(const float* sorted, int* src, uint32_t* e, uint32
     if (c <= k - 1) f = c;
     else l = c;
   }
-  if (l - f <= 3) {   // the last elements by insertion sort (stable)
+  {   // the last elements by insertion sort (stable); after the depth limit, all that are left, so
+      // that the first k are chosen whatever the order among them
     int to[NJ];
 #pragma unroll
     for (int i = 0; i < NJ; ++i) {
