@@ -93,3 +93,47 @@ def test_mlp_swiglu_equals_module(shape, gpu):
         assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.nan_to_num(), ref.nan_to_num())
         assert mlp_swiglu(mlp, h.float()) is None
     assert mlp_swiglu(mlp, h) is None
+
+
+def test_mlp_hooks_and_overrides_see_their_calls(gpu):
+    """Both short cuts leave the MLP to its own call where a hook or another forward would see it, and one
+    of its linears where only that one has them."""
+    from types import SimpleNamespace
+    from bolt3_amd import Bolt3Decoder, HybridLM
+    from bolt3_amd.layers import MLP, mlp_rows, mlp_swiglu
+    mlp = MLP(dict(dim=64, intermediate=128)).to(gpu).to(BF)
+    blk = SimpleNamespace(norm2=torch.nn.Identity(), mlp=mlp)
+    dec = Bolt3Decoder(HybridLM(vocab_size=8, dim=64, num_layers=0, num_heads=1, num_kv_heads=1, intermediate=8,
+                                layer_types=[]).to(gpu))
+    few, many = (torch.randn(*s, 64, device=gpu).to(BF) for s in ((3, 1), (2, 40)))
+    seen = []
+
+    def calls(m):
+        """The calls of m that a step and a prompt make, with and without the few-row form."""
+        n = []
+        for dec.fuse_mlp in (False, True):
+            for x in (few, many):
+                seen.clear()
+                dec._mlp(blk, x)
+                n.append(sum(s is m for s in seen))
+        return n
+
+    def note(m, *_):
+        seen.append(m)
+
+    with torch.no_grad():
+        assert mlp_swiglu(mlp, many) is not None and mlp_rows(mlp, few, few) is not None
+        hook = torch.nn.modules.module.register_module_forward_hook(note)
+        try:
+            assert calls(mlp) == [1, 1, 1, 1] and calls(mlp.up_proj) == [1, 1, 1, 1]
+        finally:
+            hook.remove()
+        for m in (mlp, mlp.down_proj):
+            hook = m.register_forward_pre_hook(note)
+            assert calls(m) == [1, 1, 1, 1]
+            hook.remove()
+            own = type(m).forward.__get__(m)
+            m.forward = lambda x, m=m, own=own: (note(m), own(x))[1]
+            assert calls(m) == [1, 1, 1, 1]
+            del m.forward
+        assert calls(mlp) == [0, 0, 0, 0]

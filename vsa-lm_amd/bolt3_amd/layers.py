@@ -104,12 +104,20 @@ class MLP(nn.Module):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
+def _untouched(m: nn.Module) -> bool:
+    """Calling m is nothing but its class's forward: no hook of its own or of all modules, no forward set
+    on the instance, not compiled.  What replaces a module's call asks for this, so that hooks and
+    overrides see the calls they saw."""
+    return not (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ or
+                m._compiled_call_impl is not None or torch.nn.modules.module._has_any_global_hook())
+
+
 MLP_ROWS = 16   # rows bolt3_rows_linear takes; the library's products are the faster ones above
 
 
 def _plain_linear(m: nn.Module, x: torch.Tensor) -> bool:
     """A linear layer that is nothing but its bf16 weight on x's device, rows as the kernel reads them."""
-    return (type(m) is nn.Linear and m.bias is None and not m._forward_hooks and not m._forward_pre_hooks and
+    return (type(m) is nn.Linear and m.bias is None and _untouched(m) and
             type(m.weight) in (nn.Parameter, torch.Tensor) and m.weight.dtype == torch.bfloat16 and
             m.weight.device == x.device and m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0 and
             m.in_features % 32 == 0 and m.out_features % 16 == 0)
@@ -118,15 +126,14 @@ def _plain_linear(m: nn.Module, x: torch.Tensor) -> bool:
 def mlp_rows(mlp: nn.Module, h: torch.Tensor, res: torch.Tensor) -> torch.Tensor | None:
     """res + mlp(h) for the few rows of a one-token decode step, in two launches that stream the weights
     once (gate, up and SwiGLU; down and the residual), with the roundings of the module's own ops.
-    None where it does not apply: gradients, autocast or hooks, other modules, dtypes or layouts,
-    more than MLP_ROWS rows."""
+    None where it does not apply: gradients, autocast, hooks or overrides, other modules, dtypes or
+    layouts, more than MLP_ROWS rows."""
     D = h.shape[-1]
     M = h.numel() // D if D else 0
     if (type(mlp) is not MLP or not 0 < M <= MLP_ROWS or not h.is_cuda or h.dtype != torch.bfloat16 or
             res.dtype != h.dtype or res.shape != h.shape or res.device != h.device or
             type(h) is not torch.Tensor or type(res) is not torch.Tensor or torch.is_grad_enabled() or
-            torch.is_autocast_enabled(h.device.type) or mlp._forward_hooks or mlp._forward_pre_hooks or
-            torch.nn.modules.module._has_any_global_hook()):
+            torch.is_autocast_enabled(h.device.type) or not _untouched(mlp)):
         return None
     gate, up, down = mlp.gate_proj, mlp.up_proj, mlp.down_proj
     if not (_plain_linear(gate, h) and _plain_linear(up, h) and _plain_linear(down, h)):
@@ -155,10 +162,10 @@ def mlp_rows(mlp: nn.Module, h: torch.Tensor, res: torch.Tensor) -> torch.Tensor
 
 def mlp_swiglu(mlp: nn.Module, h: torch.Tensor) -> torch.Tensor | None:
     """mlp(h) with SwiGLU as one pass over the two projections' outputs instead of the module's two (the
-    same roundings); None where it does not apply (gradients, autocast, another MLP, not bf16)."""
+    same roundings); None where it does not apply (gradients, autocast, hooks on the MLP or on all modules,
+    an overridden forward, another MLP, not bf16)."""
     if (type(mlp) is not MLP or not h.is_cuda or h.dtype != torch.bfloat16 or type(h) is not torch.Tensor or
-            torch.is_grad_enabled() or torch.is_autocast_enabled(h.device.type) or mlp._forward_hooks or
-            mlp._forward_pre_hooks):
+            torch.is_grad_enabled() or torch.is_autocast_enabled(h.device.type) or not _untouched(mlp)):
         return None
     g, u = mlp.gate_proj(h), mlp.up_proj(h)
     if (g.dtype != torch.bfloat16 or u.dtype != g.dtype or u.shape != g.shape or u.device != g.device or
