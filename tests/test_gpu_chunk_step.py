@@ -3,7 +3,9 @@ every head ratio's kernel, query counts and window lengths at the edges of the 3
 and without sinks, slots (masked ones among them), an older window segment and M_res.
 
 The kernel rounds the probabilities, the attention, the readout and their sum to bf16 (2^-8 of each,
-the probabilities' against the values' magnitudes) and splits M_res into 16 mantissa bits."""
+the probabilities' against the values' magnitudes) and splits M_res into 16 mantissa bits.
+
+And against attn_kernel, which M_res and outputs off their alignment take: the same bits."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -77,3 +79,51 @@ def test_chunk_step_matches_fp32(G, HD, t, old, a_len, slots, sinks, readout, gp
     bound = 1.1 * 2.0 ** -8 * (mass + att.abs() + rd.abs() + ref.abs()) + 1e-4 * (mass + rd.abs())
     worst = float(((got - ref).abs() / bound).max())
     assert worst <= 1.0, worst
+
+
+def _step(gpu, G, HD, t, old, a_len, off, score_round=0):
+    """One chunk step, its M_res off floats into a buffer and its output rows off elements apart from a
+    multiple of four; every field in use, the first slots masked."""
+    from bolt3_amd import _abi as A
+    B, HKV, S, cap = 2, 2, 128, 512
+    H = G * HKV
+    g = torch.Generator(device=gpu).manual_seed(t + old + HD)
+
+    def r(*s, dt=BF):
+        return torch.randn(*s, generator=g, device=gpu).to(dt)
+
+    q, q_raw, eta = r(B, H, t, HD), r(B, H, t, HD), torch.tanh(r(B, H, t, dt=torch.float32))
+    wk, wv, sk, sv = r(B, HKV, cap, HD), r(B, HKV, cap, HD), r(B * HKV, S, HD), r(B * HKV, S, HD)
+    ck, cv, m0 = r(B, HKV, 4, HD), r(B, HKV, 4, HD), 0.3 * r(B, HKV, HD, HD, dt=torch.float32)
+    bias, gamma, res_w = (torch.rand(*s, generator=g, device=gpu) for s in ((B * HKV, S), (HKV,), (HD,)))
+    bias[:, :40] = float("-inf")
+    buf = torch.zeros(m0.numel() + 4, device=gpu)
+    m = buf[off:off + m0.numel()].view(m0.shape).copy_(m0)
+    st = H * HD + off
+    y = torch.full((B * (t + 1) * st + 4,), 7.0, dtype=BF, device=gpu)[off:]
+    a = A.AttnArgs()
+    a.dtype, a.B, a.H, a.HKV, a.HD, a.S, a.C, a.n_sinks, a.mode, a.n_q = 1, B, H, HKV, HD, S, 128, 4, 1, t
+    a.score_round = score_round
+    a.q_rope, a.q_raw, a.q_sb, a.q_sh = q.data_ptr(), q_raw.data_ptr(), q.stride(0), q.stride(1)
+    a.eta, a.e_sb, a.e_sh = eta.data_ptr(), eta.stride(0), eta.stride(1)
+    a.win_k, a.win_v, a.w_sb, a.w_sh = wk.data_ptr(), wv.data_ptr(), wk.stride(0), wk.stride(1)
+    a.a_start, a.a_len, a.b_start, a.b_len = 0, a_len, 256, old + t
+    a.sink_k, a.sink_v, a.s_sb, a.s_sh, a.n_sink_keys = ck.data_ptr(), cv.data_ptr(), ck.stride(0), ck.stride(1), 4
+    a.slot_k, a.slot_v, a.slot_bias, a.slot_step, a.has_slots = sk.data_ptr(), sv.data_ptr(), bias.data_ptr(), 0, 1
+    a.m_res, a.m_step, a.gamma, a.res_w, a.eps = m.data_ptr(), 0, gamma.data_ptr(), res_w.data_ptr(), 1e-6
+    a.y, a.y_sb, a.y_st = y.data_ptr(), (t + 1) * st, st
+    A.call("bolt3_chunk_attn", a, gpu)
+    out = y[:B * (t + 1) * st].view(B, t + 1, st)
+    assert bool((out[:, t] == 7).all()) and bool((out[..., H * HD:] == 7).all())
+    return out[:, :t, :H * HD]
+
+
+@pytest.mark.parametrize("G,HD", [(1, 64), (1, 128), (2, 64), (2, 128), (4, 64), (4, 128), (8, 64), (8, 128)])
+@pytest.mark.parametrize("t,old,a_len", [(128, 0, 128), (1, 5, 0), (33, 31, 129), (100, 127, 200)])
+def test_chunk_step_gives_attn_kernels_bits(G, HD, t, old, a_len, gpu):
+    """A state's later slot decisions follow every rounding of the layers below, so which kernel takes a
+    chunk step must not show."""
+    print(f"[case] chunk step bits G={G} HD={HD} t={t}", flush=True)
+    staged = _step(gpu, G, HD, t, old, a_len, 0)
+    for off in (1, 2):
+        assert torch.equal(_step(gpu, G, HD, t, old, a_len, off), staged)

@@ -1443,9 +1443,12 @@ static int launch_attn(const b3_attn_args& a, hipStream_t st) {
   if constexpr (St<T>::is_bf16) {
     // the decoder's chunk step on the forward's kernel: 128 tokens of 4 sequences of a Qwen3-4B-shape
     // layer take 34 us against 81 in attn_kernel, whose 32-key tiles go through registers with two
-    // barriers each (it keeps head ratios whose wavefronts the tiles do not divide over)
+    // barriers each (it keeps head ratios whose wavefronts the tiles do not divide over, and M_res and
+    // outputs that may not be read and written in 16 and 8 bytes; both give the same bits)
     const int nw = nthreads / 64;
-    if (a.mode == 1 && (!a.m_res || !a.m_split) && (!a.has_slots || a.S == 128) && a.n_sink_keys <= KB &&
+    const bool wide = reinterpret_cast<uintptr_t>(a.m_res) % 16 == 0 && reinterpret_cast<uintptr_t>(a.y) % 8 == 0 &&
+                      a.y_sb % 4 == 0 && a.y_st % 4 == 0;
+    if (a.mode == 1 && wide && (!a.m_res || !a.m_split) && (!a.has_slots || a.S == 128) && a.n_sink_keys <= KB &&
         (nw == 2 || nw == 4 || nw == 8)) {
       if (a.score_round) launch_fwd2<HD, true, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
       else launch_fwd2<HD, false, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
