@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from bolt3_amd import Bolt3Attn
-from bolt3_amd.bolt3 import _n_groups, _step_groups
+from bolt3_amd.bolt3 import _group_count, _n_groups, _step_groups
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CFG = dict(dim=64, num_heads=4, num_kv_heads=2, head_dim=16, rope_theta=1e4, eps=1e-6, qk_norm=True)
@@ -44,6 +44,12 @@ def test_step_groups_of_the_benchmark_forward():
 
 def test_short_sequences_take_fewer_groups():
     assert [_n_groups(n) for n in (1, 11, 12, 21, 22, 111, 112)] == [1, 1, 2, 2, 3, 3, 4]
+
+
+def test_one_group_where_the_decisions_crowd_the_chip():
+    """A third of 256 compute units: 86 workgroups.  Long sequences keep their groups."""
+    assert [_group_count(n, 86, 256) for n in (1, 12, 21, 22, 112)] == [1, 1, 1, 3, 4]
+    assert [_group_count(n, 85, 256) for n in (1, 12, 21, 22, 112)] == [1, 2, 2, 3, 4]
 
 
 def test_packed_parameters_follow_in_place_updates():

@@ -71,12 +71,19 @@ def _wait_started(dev: torch.device, counter: torch.Tensor, target: int) -> None
 # The forward's consolidation steps are issued in this many groups, so that the slot field and
 # readout of early chunks run while the chain still decides later steps.
 CHAIN_GROUPS = 3
-# A group costs the host about 85 us (three chain launches on two streams, the attention, o_proj),
-# and a step about 17 us of chain: short sequences, whose forward is bound by the host's launches,
-# take fewer.  Forward of a Qwen3-4B-shape layer with 1 / 2 / 3 groups, us: 5 steps (1 x 777 tokens)
-# 309 / 403 / 480; 9 steps (1 x 1400) 359 / 435 / 517, (4 x 1400) 570 / 562 / 600; 14 steps (1 x 2000)
-# 470 / 466 / 563, (4 x 2000) 775 / 704 / 749; 22 steps (1 x 3000) 670 / 620 / 614; 30 steps
-# (4 x 4096) 1594 / 1354 / 1297.
+# A group costs the host about 85 us (three chain launches on two streams, the attention, o_proj) and
+# the device a copy and smaller products, and a step about 17 us of chain: short sequences take fewer.
+# Forward of a Qwen3-4B-shape layer with 1 / 2 / 3 groups, us:
+#    9 steps (T = 1300): B = 1 365 / 418 / 486, B = 8 795 / 842 / 883, B = 16 1538 / 1525 / 1552
+#   11 steps (T = 1600): B = 1 415 / 421 / 489, B = 8 946 / 1021 / 1049, B = 16 1759 / 1880 / 1903
+#   14 steps (T = 2000): B = 1 477 / 465 / 501, B = 4 738 / 702 / 750, B = 8 1091 / 1183 / 1177
+#   20 steps (T = 2800): B = 1 636 / 600 / 594, B = 4 993 / 972 / 1045, B = 8 1730 / 1700 / 1803
+#   30 steps (T = 4096): B = 4 1594 / 1354 / 1297
+# (products of some row counts fill the chip better than their neighbours', so single sizes differ by
+# 5 % either way).  Where the slot decisions' workgroups hold a third of the compute units or more, a
+# product beside them takes most of the time that it would save, and one group is enough up to the
+# same line: B = 12 17 steps 1962 / 2161 / 2037, B = 16 13 steps 1922 / 2150 / 2050, 17 steps 2480 /
+# 2793 / 2581, 20 steps 3010 / 3215 / 3420, B = 24 14 steps 3251 / 3560 / 3519.
 ONE_GROUP_STEPS, TWO_GROUP_STEPS = 11, 21
 # ... and at least one group per this many steps, so that the work left after the last group's
 # slot decisions (its M_res updates, attention and o_proj) stays short on long sequences
@@ -93,6 +100,13 @@ def _n_groups(n_steps: int) -> int:
     if n_steps <= TWO_GROUP_STEPS:
         return 1 if n_steps <= ONE_GROUP_STEPS else 2
     return max(CHAIN_GROUPS, round(n_steps / GROUP_STEPS))
+
+
+def _group_count(n_steps: int, decide_wgs: int, n_cus: int) -> int:
+    """Step groups of a forward whose slot decisions take decide_wgs of the device's n_cus compute units."""
+    if 3 * decide_wgs >= n_cus and n_steps <= TWO_GROUP_STEPS:
+        return 1
+    return _n_groups(n_steps)
 
 
 def _step_groups(n: int, k: int) -> list[tuple[int, int]]:
@@ -363,7 +377,7 @@ class Bolt3Attn(nn.Module):
         # bf16: the chain's steps go out in groups; the slot decisions of a group run on one side
         # stream, its Gershgorin scales and M_res updates on another, and the main stream adds the
         # slot field and readout of a group's chunks as soon as that group is done
-        groups = _step_groups(n_cons, _n_groups(n_cons) if split else 1) if n_cons > 0 else []
+        groups = _step_groups(n_cons, _group_count(n_cons, bh, _n_cus(dev)) if split else 1) if n_cons > 0 else []
         done = []   # per group: event after its M_res updates
         # the first group's slot decisions hold their compute units before the q projection, a
         # GEMM whose grid covers the whole chip, is issued: otherwise most of them wait for its end
