@@ -81,7 +81,7 @@ def test_chunk_step_matches_fp32(G, HD, t, old, a_len, slots, sinks, readout, gp
     assert worst <= 1.0, worst
 
 
-def _step(gpu, G, HD, t, old, a_len, off, score_round=0):
+def _step(gpu, G, HD, t, old, a_len, off):
     """One chunk step, its M_res off floats into a buffer and its output rows off elements apart from a
     multiple of four; every field in use, the first slots masked."""
     from bolt3_amd import _abi as A
@@ -102,8 +102,7 @@ def _step(gpu, G, HD, t, old, a_len, off, score_round=0):
     st = H * HD + off
     y = torch.full((B * (t + 1) * st + 4,), 7.0, dtype=BF, device=gpu)[off:]
     a = A.AttnArgs()
-    a.dtype, a.B, a.H, a.HKV, a.HD, a.S, a.C, a.n_sinks, a.mode, a.n_q = 1, B, H, HKV, HD, S, 128, 4, 1, t
-    a.score_round = score_round
+    a.dtype, a.B, a.H, a.HKV, a.HD, a.S, a.C, a.n_sinks, a.mode, a.n_q, a.score_round = 1, B, H, HKV, HD, S, 128, 4, 1, t, 0
     a.q_rope, a.q_raw, a.q_sb, a.q_sh = q.data_ptr(), q_raw.data_ptr(), q.stride(0), q.stride(1)
     a.eta, a.e_sb, a.e_sh = eta.data_ptr(), eta.stride(0), eta.stride(1)
     a.win_k, a.win_v, a.w_sb, a.w_sh = wk.data_ptr(), wv.data_ptr(), wk.stride(0), wk.stride(1)

@@ -904,6 +904,7 @@ struct Fwd2Smem {
 template <int HD, int NW, int NPS, bool SR, bool CH>
 __global__ void __launch_bounds__(64 * NW, NPS == 2 ? 2 : 1) attn_fwd2_kernel(b3_attn_args a, int QW) {
   static_assert(NPS == 2 || NPS == 3, "two or three pair slots");
+  static_assert(!(SR && CH), "a chunk step's scores are not rounded");
   using Sm = Fwd2Smem<HD, NPS>;
   __shared__ Sm sm;
   constexpr int NDB = HD / 32, NP = HD / 8;
@@ -1106,7 +1107,7 @@ __global__ void __launch_bounds__(64 * NW, NPS == 2 ? 2 : 1) attn_fwd2_kernel(b3
       for (int r4 = 0; r4 < 4; ++r4)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float x = mul_rn(SR ? round_bf(sc[4 * r4 + e]) : sc[4 * r4 + e], scale);
+          const float x = mul_rn(sc[4 * r4 + e], scale);
           sc[4 * r4 + e] = biased ? add_rn(x, b4[r4][e]) : x;
         }
     } else {
@@ -1443,22 +1444,24 @@ static int launch_attn(const b3_attn_args& a, hipStream_t st) {
   if constexpr (St<T>::is_bf16) {
     // the decoder's chunk step on the forward's kernel: 128 tokens of 4 sequences of a Qwen3-4B-shape
     // layer take 34 us against 81 in attn_kernel, whose 32-key tiles go through registers with two
-    // barriers each (it keeps head ratios whose wavefronts the tiles do not divide over, and M_res and
-    // outputs that may not be read and written in 16 and 8 bytes; both give the same bits)
+    // barriers each (it keeps head ratios whose wavefronts the tiles do not divide over, M_res and
+    // outputs that may not be read and written in 16 and 8 bytes, and rounded scores, which no
+    // decoder asks for; both give the same bits)
     const int nw = nthreads / 64;
     const bool wide = reinterpret_cast<uintptr_t>(a.m_res) % 16 == 0 && reinterpret_cast<uintptr_t>(a.y) % 8 == 0 &&
                       a.y_sb % 4 == 0 && a.y_st % 4 == 0;
-    if (a.mode == 1 && wide && (!a.m_res || !a.m_split) && (!a.has_slots || a.S == 128) && a.n_sink_keys <= KB &&
+    if (a.mode == 1 && wide && !a.score_round && (!a.m_res || !a.m_split) && (!a.has_slots || a.S == 128) && a.n_sink_keys <= KB &&
         (nw == 2 || nw == 4 || nw == 8)) {
-      if (a.score_round) launch_fwd2<HD, true, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
-      else launch_fwd2<HD, false, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
+      launch_fwd2<HD, false, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
       return (int)hipGetLastError();
     }
   }
   if constexpr (!St<T>::is_bf16) {
     // fp32: one query tile per head and workgroup where two would leave CUs without one (a wavefront's
     // own work is the same, and so are the bits).  1 x 1024 tokens, 3 kv heads of 3: 96 workgroups for 48.
-    if (QW == 2 && G >= 2 && (long long)grid.x * grid.y * grid.z < 256) {
+    const int n_cu = cu_count();
+    if (n_cu < 0) return -n_cu;
+    if (QW == 2 && G >= 2 && (long long)grid.x * grid.y * grid.z < n_cu) {
       hipLaunchKernelGGL((attn_kernel<T, HD>), dim3((qlen + 31) / 32, grid.y, grid.z), dim3(64 * G), 0, st, a, 1);
       return (int)hipGetLastError();
     }
