@@ -114,7 +114,8 @@ StaticKV = AnchorCache
 
 
 def _zeros(device, dtype, *shapes):
-    """Zero tensors of the given shapes, cleared in one launch."""
+    """Zero tensors of the given shapes, cleared by one multi-tensor fill (several launches where they
+    are large)."""
     out = [torch.empty(s, dtype=dtype, device=device) for s in shapes]
     torch._foreach_zero_(out)
     return out
@@ -205,7 +206,7 @@ class Bolt3LayerState(MutableMapping):
         self.cap = 4 * C
         bh = B * HKV
         win, sink, slot = (B, HKV, self.cap, HD), (B, HKV, N_SINKS, HD), (bh, S, HD)
-        # one zero fill per dtype instead of one per tensor (some 4 us each, in every layer of a prefill)
+        # a multi-tensor fill per dtype instead of a fill per tensor (some 4 us each, in every layer of a prefill)
         self.win_kr, self.win_kp, self.win_v, self.sink_k, self.sink_v, ak, av, self.slot_k = _zeros(
             device, dtype, win, win, win, sink, sink, slot, slot, slot)
         self.win_b, self.win_pos, util, pm, self.slot_bias = _zeros(

@@ -525,7 +525,9 @@ struct FwdBlock {
   const uint16_t* v;
   const float* bias;   // null: no bias
   int nvalid;
-  int kpos;            // current-chunk block: index of its first key within the chunk; else -1
+  // the block's place for the causal mask.  attn_fwd_kernel: a current-chunk block's first key within
+  // the chunk, else -1.  attn_fwd2_kernel: that key relative to query 0 (negative before it), else ALL
+  int kpos;
 };
 
 template <int HD, int IPT>
@@ -1239,7 +1241,7 @@ __global__ void __launch_bounds__(64 * NW, NPS == 2 ? 2 : 1) attn_fwd2_kernel(b3
     }
     const int i0 = 2 * pr, i1 = 2 * pr + 1;
     const FwdBlock f0 = block(i0);
-    const bool do0 = f0.kpos <= wave_q0 + 31;   // the wave's queries all precede the block
+    const bool do0 = f0.kpos <= wave_q0 + 31;   // else the wave's queries all precede the block
     const bool has1 = i1 < nb;
     const FwdBlock f1 = block(has1 ? i1 : i0);
     const bool do1 = has1 && f1.kpos <= wave_q0 + 31;
