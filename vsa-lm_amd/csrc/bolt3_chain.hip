@@ -1424,7 +1424,8 @@ __global__ void __launch_bounds__(DT) decide_kernel(b3_chain_args a) {
     if (__builtin_expect(nf == 0, 0)) {
       // score = unbiased variance of normalize(v), one thread per token: the scores order the slots and
       // every later tie follows that order, so their bits matter (four threads per token with the sums
-      // handed on in order took 21 us instead of 31, but differed by an ulp in 9 of 2000 tokens)
+      // handed on in order took 21 us instead of 31, but differed by an ulp in 9 of 2000 tokens, for a
+      // reason not found)
       const int j = tid;
       if (j < l) {
         const T* vr = v + (long long)j * HD;

@@ -10,7 +10,8 @@
 // columns per workgroup), 18 us at the SmolLM shape with 4 x 1100.  It takes the place of about 25
 // elementwise and reduction launches, which bound the second (forward and backward 1.59 -> 1.23
 // ms); in the first their column sums of the projection gradient ran beside its two products,
-// slowing them, and for 55 us after them.
+// slowing them, and for 55 us after them.  Where q, k and v have biases (all 6192 columns of the
+// first shape instead of 40) forward and backward take 5.26-5.28 ms against 5.32-5.45 with those sums.
 #include "bolt3_common.h"
 #include "bolt3_amd.h"
 
