@@ -150,10 +150,11 @@ def layer_backward(mod, x: torch.Tensor, tr: dict, d_out: torch.Tensor, dt: torc
     Two streams.  This one: the o_proj products, the readout's backward, the chain's token
     statistics, the attention's backward, the chain's slot recursion and token gradients, the
     key / value part of the head backward, the small parameters' sums and the projections'
-    products.  The side stream: the chain's M_res recursion, a few long-lived workgroups that run beside the attention's backward
-    (this stream holds the attention until they are resident, bolt3_wait_count), then the query
-    part of the head backward beside the chain's slot recursion and token gradients.  Every buffer the side stream touches is allocated on this stream and held here
-    until this stream has waited for the side stream's last kernel."""
+    products.  The side stream: the chain's M_res recursion, a few long-lived workgroups that run
+    beside the attention's backward (this stream holds the attention until they are resident,
+    bolt3_wait_count), then the query part of the head backward beside the chain's slot recursion
+    and token gradients.  Every buffer the side stream touches is allocated on this stream and held
+    here until this stream has waited for the side stream's last kernel."""
     from .bolt3 import WAIT_POLLS, _n_cus, _started_counter   # (bolt3 imports this module)
     b, T, D = x.shape
     H, HKV, HD, S, C = mod.H, mod.HKV, mod.HD, mod.S, mod.C

@@ -1452,8 +1452,8 @@ static int launch_attn(const b3_attn_args& a, hipStream_t st) {
     const int nw = nthreads / 64;
     const bool wide = reinterpret_cast<uintptr_t>(a.m_res) % 16 == 0 && reinterpret_cast<uintptr_t>(a.y) % 8 == 0 &&
                       a.y_sb % 4 == 0 && a.y_st % 4 == 0;
-    if (a.mode == 1 && wide && !a.score_round && (!a.m_res || !a.m_split) && (!a.has_slots || a.S == 128) && a.n_sink_keys <= KB &&
-        (nw == 2 || nw == 4 || nw == 8)) {
+    if (a.mode == 1 && wide && !a.score_round && (!a.m_res || !a.m_split) && (!a.has_slots || a.S == 128) &&
+        a.n_sink_keys <= KB && (nw == 2 || nw == 4 || nw == 8)) {
       launch_fwd2<HD, false, true>(a, G, nw, qlen, 1, grid, nthreads, QW, st);
       return (int)hipGetLastError();
     }
